@@ -1,7 +1,7 @@
 // Full-attention layers of the hybrid trunk and of the MTP draft head
 // (Qwen3.5 gated attention) on gfx950.
 //
-//   attn_qk_kernel       one wave per (token, head): RMSNorm of q and k over
+//   attn_qk_kernel       one wave per token and group of heads: RMSNorm of q and k over
 //                        the head dim (y = x / rms(x) * w), the rotary
 //                        embedding of the first `rot` dims (rotate-half form,
 //                        angle pos * base^(-2i/rot)), q to [B, T, Hq, D]; k and
@@ -80,63 +80,132 @@ __device__ __forceinline__ int first_pos(const int32_t* pos0, int b, int T, int 
   return min(max(pos0[b], 0), cap - T);
 }
 
-template <int D>
+// EPL bf16 elements of a row at any 2-byte address, as one load / store (callers
+// may pass rows at any element offset; the hardware takes unaligned dwords).
+template <int EPL>
+struct RowVec {
+  typedef uint16_t type __attribute__((ext_vector_type(EPL), aligned(2)));
+};
+
+// One wave takes NH heads of one token (q heads, then k, then v), the last
+// wave of a token the rest.  The rotary angles depend on the token and the
+// lane only, so exp2 and sincos -- most of the arithmetic, computed per head
+// it bounded the kernel at 70.6 us for 4096 tokens of 16 + 2 x 4 heads --
+// run once for the NH heads, whose rows are all loaded before the first is
+// used and whose chains overlap.  A wave with more heads runs longer, so few
+// tokens take few heads a wave (graph-replayed, us, NH = 1 / 3 / 6):
+//   1 token 5.7 / 6.8 / 7.9, 128 tokens 6.9 / 7.2 / 8.3, 256 8.7 / 7.8 / 8.6,
+//   512 12.4 / 9.8 / 9.6, 1024 19.5 / 13.5 / 12.6, 4096 59.1 / 33.2 / 28.3
+// (100 MB: 3.6 TB/s).
+template <int D, int NH>
 __global__ __launch_bounds__(256) void attn_qk_kernel(const QkParams p) {
   constexpr int EPL = D / 64;  // elements per lane
+  typedef typename RowVec<EPL>::type vec;
   const int lane = threadIdx.x & 63;
-  const int64_t item = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int heads = p.Hq + 2 * p.Hkv;  // q heads, k heads, v heads
-  if (item >= static_cast<int64_t>(p.B) * p.T * heads) return;  // wave-uniform
-  const int h = static_cast<int>(item % heads);
-  const int64_t bt = item / heads;
+  const uint32_t per_tok = (heads + NH - 1) / NH;
+  const uint32_t item = blockIdx.x * 4u + wave;
+  const uint32_t bt = item / per_tok;
+  if (bt >= static_cast<uint32_t>(p.B) * p.T) return;  // wave-uniform
+  const int h0 = static_cast<int>(item % per_tok) * NH;
   const int t = static_cast<int>(bt % p.T), b = static_cast<int>(bt / p.T);
-  const int pos = first_pos(p.pos0, b, p.T, p.cap) + t;
   const int d0 = EPL * lane;
 
-  const uint16_t* src;
-  if (h < p.Hq) src = p.qg + bt * p.qg_ld + h * 2 * D;
-  else if (h < p.Hq + p.Hkv) src = p.kn + bt * p.kv_ld + (h - p.Hq) * D;
-  else src = p.vn + bt * p.kv_ld + (h - p.Hq - p.Hkv) * D;
-  float x[EPL];
+  vec raw[NH];
 #pragma unroll
-  for (int e = 0; e < EPL; ++e) x[e] = bf16_to_f32(src[d0 + e]);
-
-  if (h >= p.Hq + p.Hkv) {  // v: into the cache as is
-    uint16_t* dst = p.vc + ((static_cast<int64_t>(b) * p.Hkv + (h - p.Hq - p.Hkv)) * p.cap + pos) * D;
-#pragma unroll
-    for (int e = 0; e < EPL; ++e) dst[d0 + e] = src[d0 + e];
-    return;
+  for (int n = 0; n < NH; ++n) {
+    const int h = min(h0 + n, heads - 1);
+    const uint16_t* src;
+    if (h < p.Hq) src = p.qg + bt * p.qg_ld + h * 2 * D;
+    else if (h < p.Hq + p.Hkv) src = p.kn + bt * p.kv_ld + (h - p.Hq) * D;
+    else src = p.vn + bt * p.kv_ld + (h - p.Hq - p.Hkv) * D;
+    raw[n] = *reinterpret_cast<const vec*>(src + d0);
   }
-  // RMSNorm, rounded to bf16 (the norm's output dtype)
-  float ss = 0.0f;
+  // norm weights as raw bits (converted after every load is issued); a single
+  // head's wave loads its own kind's only
+  uint32_t qwr[EPL], kwr[EPL];
+  const void* qwp = NH > 1 || h0 < p.Hq ? p.qw : p.kw;
 #pragma unroll
-  for (int e = 0; e < EPL; ++e) ss += x[e] * x[e];
-  const float r = rsqrtf(wave_sum(ss) / D + p.eps);
-  const void* w = h < p.Hq ? p.qw : p.kw;
-#pragma unroll
-  for (int e = 0; e < EPL; ++e) x[e] = bf16_to_f32(f32_to_bf16(x[e] * r * load_any(w, p.wdt, d0 + e)));
+  for (int e = 0; e < EPL; ++e) {
+    if (p.wdt == GDN_DTYPE_F32) {
+      qwr[e] = static_cast<const uint32_t*>(qwp)[d0 + e];
+      if (NH > 1) kwr[e] = static_cast<const uint32_t*>(p.kw)[d0 + e];
+    } else {
+      qwr[e] = static_cast<const uint16_t*>(qwp)[d0 + e];
+      if (NH > 1) kwr[e] = static_cast<const uint16_t*>(p.kw)[d0 + e];
+    }
+  }
+  const int pos = first_pos(p.pos0, b, p.T, p.cap) + t;
+
   // rotary embedding of dims [0, rot): d < half pairs with d + half
   const int half = p.rot / 2;
   const int shift = half / EPL;  // lanes between partners
-  float y[EPL];
+  const bool lower = d0 < half;
+  const int partner = lower ? lane + shift : lane - shift;
+  float sn[EPL], cs[EPL];
 #pragma unroll
   for (int e = 0; e < EPL; ++e) {
-    const bool lower = d0 < half;
-    const float other = __shfl(x[e], lower ? lane + shift : lane - shift, 64);
-    if (d0 < p.rot) {
+    sn[e] = 0.0f;
+    cs[e] = 1.0f;
+  }
+  if (d0 < p.rot && h0 < p.Hq + p.Hkv) {
+#pragma unroll
+    for (int e = 0; e < EPL; ++e) {
       const int i = half > 0 ? (d0 + e) % half : 0;
       const float inv_freq = exp2f(-2.0f * static_cast<float>(i) / static_cast<float>(p.rot) * p.log2_base);
-      float sn, cs;
-      sincosf(static_cast<float>(pos) * inv_freq, &sn, &cs);
-      y[e] = lower ? x[e] * cs - other * sn : x[e] * cs + other * sn;
-    } else {
-      y[e] = x[e];
+      sincosf(static_cast<float>(pos) * inv_freq, &sn[e], &cs[e]);
     }
   }
-  uint16_t* dst = h < p.Hq ? p.q + (bt * p.Hq + h) * D
-                           : p.kc + ((static_cast<int64_t>(b) * p.Hkv + (h - p.Hq)) * p.cap + pos) * D;
+  auto weight = [&](uint32_t u) {
+    return p.wdt == GDN_DTYPE_F32 ? __uint_as_float(u)
+                                  : (p.wdt == GDN_DTYPE_BF16 ? bf16_to_f32(static_cast<uint16_t>(u))
+                                                             : f16_to_f32(static_cast<uint16_t>(u)));
+  };
+  float qw[EPL], kw[EPL];
 #pragma unroll
-  for (int e = 0; e < EPL; ++e) dst[d0 + e] = f32_to_bf16(y[e]);
+  for (int e = 0; e < EPL; ++e) {
+    qw[e] = weight(qwr[e]);
+    kw[e] = NH > 1 ? weight(kwr[e]) : qw[e];
+  }
+
+  // the heads' chains (sum, norm, exchange) carry no branch, so they overlap
+  float r[NH];
+#pragma unroll
+  for (int n = 0; n < NH; ++n) {
+    float ss = 0.0f;
+#pragma unroll
+    for (int e = 0; e < EPL; ++e) {
+      const float x = bf16_to_f32(raw[n][e]);
+      ss += x * x;
+    }
+    r[n] = rsqrtf(wave_sum(ss) / D + p.eps);
+  }
+  vec out[NH];
+#pragma unroll
+  for (int n = 0; n < NH; ++n) {
+#pragma unroll
+    for (int e = 0; e < EPL; ++e) {
+      // RMSNorm, rounded to bf16 (the norm's output dtype)
+      const float x = bf16_to_f32(f32_to_bf16(bf16_to_f32(raw[n][e]) * r[n] * (h0 + n < p.Hq ? qw[e] : kw[e])));
+      const float other = __shfl(x, partner, 64);
+      const float y = d0 < p.rot ? (lower ? x * cs[e] - other * sn[e] : x * cs[e] + other * sn[e]) : x;
+      out[n][e] = f32_to_bf16(y);
+    }
+  }
+#pragma unroll
+  for (int n = 0; n < NH; ++n) {
+    const int h = h0 + n;
+    if (h >= heads) return;  // wave-uniform
+    if (h < p.Hq) {
+      *reinterpret_cast<vec*>(p.q + (static_cast<int64_t>(bt) * p.Hq + h) * D + d0) = out[n];
+    } else {
+      const bool is_k = h < p.Hq + p.Hkv;  // v goes into the cache as is
+      const int hkv = h - p.Hq - (is_k ? 0 : p.Hkv);
+      *reinterpret_cast<vec*>((is_k ? p.kc : p.vc) + ((static_cast<int64_t>(b) * p.Hkv + hkv) * p.cap + pos) * D + d0) =
+          is_k ? out[n] : raw[n];
+    }
+  }
 }
 
 // ------------------------------------------------------------ attn_fwd
@@ -951,11 +1020,17 @@ extern "C" int gdn_attn_qk(const void* qg, int64_t qg_ld, const void* k_new, con
   p.rot = static_cast<int>(rot);
   p.eps = eps;
   p.log2_base = log2f(rope_base);
-  const int64_t waves = B * T * (Hq + 2 * Hkv);
-  const dim3 grid(static_cast<unsigned>((waves + 3) / 4));
   hipStream_t st = static_cast<hipStream_t>(stream);
-  if (D == 256) hipLaunchKernelGGL(attn_qk_kernel<256>, grid, dim3(256), 0, st, p);
-  else hipLaunchKernelGGL(attn_qk_kernel<128>, grid, dim3(256), 0, st, p);
+  // heads per wave by the number of tokens (attn_qk_kernel's comment has both sides of each line)
+  auto launch = [&](auto nh) {
+    constexpr int NH = decltype(nh)::value;
+    const dim3 grid(static_cast<unsigned>((B * T * ((Hq + 2 * Hkv + NH - 1) / NH) + 3) / 4));
+    if (D == 256) hipLaunchKernelGGL((attn_qk_kernel<256, NH>), grid, dim3(256), 0, st, p);
+    else hipLaunchKernelGGL((attn_qk_kernel<128, NH>), grid, dim3(256), 0, st, p);
+  };
+  if (B * T <= 128) launch(std::integral_constant<int, 1>{});
+  else if (B * T < 512) launch(std::integral_constant<int, 3>{});
+  else launch(std::integral_constant<int, 6>{});
   return gdn_host::check_launch("gdn_attn_qk");
 }
 

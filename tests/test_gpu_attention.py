@@ -88,6 +88,43 @@ def test_qk_prep_matches_oracle():
         assert not kc_n[b, :, untouched].any() and not vc_n[b, :, untouched].any()
 
 
+@pytest.mark.parametrize("B,T,Hq,Hkv,D,wdt", [
+    (1, 128, 10, 2, 256, torch.float32),   # one head a wave, its last size
+    (3, 43, 10, 2, 128, torch.bfloat16),   # 129 tokens: three heads a wave, 14 heads in 5 groups
+    (1, 511, 5, 1, 256, torch.float16),
+    (2, 256, 10, 2, 256, torch.bfloat16),  # 512 tokens: six heads a wave, the last with two
+    (1, 601, 4, 4, 128, torch.float32),
+])
+def test_qk_prep_head_groups(B, T, Hq, Hkv, D, wdt):
+    """The prep's head groups at their edges, with rows at an odd element
+    offset.  Norm and rotation round to bf16 once each: 2 u / sqrt(3) = 4.5e-3
+    worst, 4e-3 as in the test above (the norm's rounding is the oracle's too)."""
+    gen = torch.Generator().manual_seed(83)
+    rot, base, cap = D // 4, 1.0e7, T + 70
+    pos0 = [7 * b for b in range(B)]
+    wide = _bf16(gen, B, T, (2 * Hq + 2 * Hkv) * D + 3)
+    qw = (torch.randn(D, generator=gen) * 0.2 + 1.0).to(wdt)
+    kw = (torch.randn(D, generator=gen) * 0.2 + 1.0).to(wdt)
+    kc = torch.zeros(B, Hkv, cap, D, dtype=torch.bfloat16, device=DEV)
+    vc = torch.zeros_like(kc)
+    parts = [wide[..., 1 + lo * D:1 + hi * D] for lo, hi in ((0, 2 * Hq), (2 * Hq, 2 * Hq + Hkv),
+                                                             (2 * Hq + Hkv, 2 * Hq + 2 * Hkv))]
+    dev = [wide.to(DEV)[..., 1 + lo * D:1 + hi * D] for lo, hi in ((0, 2 * Hq), (2 * Hq, 2 * Hq + Hkv),
+                                                                   (2 * Hq + Hkv, 2 * Hq + 2 * Hkv))]
+    q = att.attn_qk(*dev, qw.to(DEV), kw.to(DEV), 1e-6, torch.tensor(pos0, dtype=torch.int32, device=DEV), kc, vc,
+                    rot, base)
+    torch.cuda.synchronize()
+    rq, _, rk, rv = oa.qk_prep(*(_np(x) for x in parts), _np(qw), _np(kw), 1e-6, pos0, rot, base, Hq, Hkv, D,
+                               round_fn=bf16_round)
+    assert _row_errs(_np(q), rq).max() < 4e-3
+    kc_n, vc_n = _np(kc), _np(vc)
+    for b in range(B):
+        sl = slice(pos0[b], pos0[b] + T)
+        assert _row_errs(kc_n[b, :, sl], rk[b].transpose(1, 0, 2)).max() < 4e-3
+        np.testing.assert_array_equal(vc_n[b, :, sl], rv[b].transpose(1, 0, 2))
+        assert not kc_n[b, :, :pos0[b]].any() and not vc_n[b, :, pos0[b] + T:].any()
+
+
 def test_rms_norm_residual_and_strided_output():
     """``gdn_rms_norm`` with a fused residual add (h = bf16(x + r), written
     out) and its output in one half of a concatenation buffer, against
