@@ -20,15 +20,17 @@
 //                        Keys may also be split over workgroups; the partial
 //                        states then go to a workspace and
 //   attn_combine_kernel  merges them.
-//   attn_prefill_kernel  long prefills (one key range, >= 512 rows per kv-head):
-//                        128-row workgroups, 32 rows per wave, 64-key K / V
-//                        blocks double-buffered in LDS (K by direct loads, V
-//                        transposed on its way in), one barrier per block.
+//   attn_prefill_kernel  long prefills (>= 512 rows per kv-head): 128-row
+//                        workgroups, 64-key K / V blocks double-buffered in
+//                        LDS (K by direct loads, V transposed on its way in),
+//                        one barrier per block; keys split likewise.
 //                        The output is multiplied by sigmoid(gate) on the way
 //                        out when a gate is given.
 //   rms_norm_kernel      the layers' RMSNorm over the hidden size, optionally of
 //                        a residual sum it also writes out.
 //   silu_mul_kernel      the MLP's silu(gate) * up.
+#include <cfloat>
+
 #include "gdn_common.hpp"
 
 namespace {
@@ -486,10 +488,10 @@ __global__ __launch_bounds__(256) void attn_fwd_kernel(const AttnParams p) {
   }
 }
 
-// Long causal prefills (one key range, at least kPrefillRows rows per kv-head):
-// a workgroup owns 128 rows, four waves of 32, so every K or V fragment a
-// wave reads from LDS feeds two 16-row MFMA tiles.  64-key blocks are double-
-// buffered in LDS and a block costs one barrier:
+// Causal prefills of at least kPrefillRows rows per kv-head: a workgroup owns
+// 128 rows in four row groups of 32, so every K or V fragment a wave reads
+// from LDS feeds two 16-row MFMA tiles.  64-key blocks are double-buffered in
+// LDS and a block costs one barrier:
 //   K  goes in by direct global -> LDS loads (each lane's 16 bytes land at
 //      16 * lane past the wave's base), rows of D bf16 whose 16-byte granules
 //      are XOR-swizzled by (key & 7), so the fragment reads of 8 consecutive
@@ -501,19 +503,46 @@ __global__ __launch_bounds__(256) void attn_fwd_kernel(const AttnParams p) {
 //      granules are XOR-swizzled by (d & 7), which keeps both the fragment
 //      reads and the 8-byte transposed writes free of bank conflicts.  (Transposed LDS reads of a [key][d]
 //      block deliver about 45 bytes per clock per CU, against 128 for 16-byte
-//      reads.)
+//      reads.)  Its loads are issued one block ahead of the transpose.
+// KG = 2 (head dim 256, whose workgroup fills a CU's LDS): eight waves, two
+// per SIMD, the two of a row group taking 32 keys of every block each with a
+// softmax state of their own, merged in LDS at the end.  One wave's MFMAs
+// then run beside the other's exponentials: a single wave issues a 16x16x32
+// MFMA every 9.6 ns at best and two share a SIMD at 7.6 ns each, with two or
+// three vector instructions per MFMA free.  Both must fit in 256 registers
+// each without a spill (a reload per block waits for every load in flight:
+// +9% per fragment), which is why two k-steps of q stay in LDS and few
+// fragments are in flight.  KG = 1 (head dim 128): four waves, and two
+// workgroups share a CU.
+// Measured at 16 query and 4 kv-heads of 256: 4096 tokens 195 -> 165 us
+// (840 TFLOP/s), 512 tokens over a 4096-token prefix in one key range 160 ->
+// 128 us; four waves with the next block's scores computed between this
+// block's exponentials, in registers enough for both, took 209 and 172 us.
+// Few rows leave CUs idle, so the keys may be split over workgroups too
+// (n_split; 512 tokens over 4096 in four ranges: 60 us with the combine).
 // The softmax max is raised only when a row's block max exceeds it by more
 // than 8 (log2 units; P stays below 2^8), which skips the rescale of the
 // output on most blocks, and only blocks that cross the diagonal or the end
 // of the keys are masked.  Workgroups with the longest key ranges go first.
-// 16 bytes per lane from global memory straight into LDS at lds_base + 16 * lane (lds_base wave-
-// uniform).  Issued from inline assembly: the compiler's wait insertion, seeing an LDS DMA in a
-// loop, would otherwise drain every LDS read with lgkmcnt(0).  It increments vmcnt like any load;
-// the caller waits for it (vmcnt(0)) before the barrier that publishes the block.
-__device__ __forceinline__ void lds_dma16(const void* gptr, uint32_t lds_base) {
-  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
+
+// A raw buffer descriptor of `bytes` bytes at `base` (wave-uniform): reads past its end return zeros.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buf_rsrc(const void* base, uint32_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, static_cast<int>(bytes), 0x00020000);
+}
+// The same descriptor as four words, for inline assembly.
+__device__ __forceinline__ u32x4 buf_words(const void* base, uint32_t bytes) {
+  const uint64_t a = reinterpret_cast<uint64_t>(base);
+  return u32x4{static_cast<uint32_t>(a), static_cast<uint32_t>(a >> 32) & 0xffffu, bytes, 0x00020000u};
+}
+
+// 16 bytes per lane from a buffer (byte offset voff) straight into LDS at lds_base + 16 * lane (rsrc and
+// lds_base wave-uniform).  Issued from inline assembly: the compiler's wait insertion, seeing an LDS DMA in
+// a loop, would otherwise drain every LDS read with lgkmcnt(0).  It increments vmcnt like any load; the
+// caller waits for it (vmcnt(0)) before the barrier that publishes the block.
+__device__ __forceinline__ void lds_dma16(u32x4 rsrc, uint32_t voff, uint32_t lds_base) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds"
                :
-               : "v"(gptr), "s"(lds_base)
+               : "v"(voff), "s"(rsrc), "s"(lds_base)
                : "memory", "m0");
 }
 
@@ -533,24 +562,39 @@ __device__ __forceinline__ float rows_sum(float x) {
   return __uint_as_float(b[0]) + __uint_as_float(b[1]);
 }
 
+// Max over the 64 lanes.
+__device__ __forceinline__ float wave_max(float x) {
+  x = fmaxf(x, dpp_f<GDN_DPP_QUAD_XOR1>(x));
+  x = fmaxf(x, dpp_f<GDN_DPP_QUAD_XOR2>(x));
+  x = fmaxf(x, dpp_f<GDN_DPP_HALF_MIRROR>(x));
+  x = fmaxf(x, dpp_f<GDN_DPP_ROW_MIRROR>(x));
+  return rows_max(x);
+}
+
 constexpr int kPrefillRows = 512;  // rows (tokens x heads of a group) per kv-head from which it is used
 constexpr int PR = 128;            // rows per workgroup
 constexpr int VTP = KB;            // Vt row stride (bf16); 16-byte granules XOR-swizzled by (d & 7)
 
-template <int D>
-__global__ __launch_bounds__(256) void attn_prefill_kernel(const AttnParams p) {
+template <int D, int KG>
+__global__ __launch_bounds__(256 * KG) void attn_prefill_kernel(const AttnParams p) {
+  constexpr int NT = 256 * KG;                // threads
   constexpr int NS = D / 32;                  // k-steps of q . k
   constexpr int NJ = D / 16;                  // 16-wide d tiles of the output
-  constexpr int KG = D / 8;                   // 16-byte granules per K row
-  constexpr int KDMA = KB * KG / 256;         // direct loads per thread and K block
-  constexpr int VPAIRS = (KB / 4) * KG / 256;  // (key quad, d octet) pairs per thread and V block
+  constexpr int KTW = 4 / KG;                 // 16-key tiles of a block per wave
+  constexpr int KSW = 2 / KG;                 // 32-key groups of a block per wave
+  constexpr int KROW = D / 8;                 // 16-byte granules per K row
+  constexpr int KDMA = KB * KROW / NT;        // direct loads per thread and K block
+  constexpr int VPAIRS = (KB / 4) * KROW / NT;  // (key quad, d octet) pairs per thread and V block
   constexpr int KSTAGE = KB * D * 2;          // bytes
   constexpr int VSTAGE = D * VTP * 2;
-  static_assert(KDMA * 256 == KB * KG && VPAIRS * 256 == (KB / 4) * KG, "block must split evenly over 256 threads");
+  static_assert(KDMA * NT == KB * KROW && VPAIRS * NT == (KB / 4) * KROW, "block must split evenly over the threads");
+  static_assert(KDMA <= NS && 4 * VPAIRS <= NS, "at most one K and one V load per k-step");
 
-  __shared__ __align__(16) unsigned char smem[2 * (KSTAGE + VSTAGE)];
+  constexpr int QL = KG == 2 ? 2 : 0;         // k-steps of q kept in LDS
+  constexpr int kMl = KG == 2 ? 8 * 128 * 4 : 0;  // the waves' (m, l) for the merge
+  __shared__ __align__(128) unsigned char smem[2 * (KSTAGE + VSTAGE) + kMl + 4 * 2 * QL * 1024];
 
-  const int b = blockIdx.z;
+  const int b = blockIdx.z, split = blockIdx.y;
   const int n_rb = gridDim.x / p.Hkv;
   const int hkv = blockIdx.x % p.Hkv;
   const int rb = n_rb - 1 - static_cast<int>(blockIdx.x) / p.Hkv;  // longest key ranges first
@@ -558,68 +602,88 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(const AttnParams p) {
   const int n_rows = p.T * g;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int rg = wave & 3, kh = wave >> 2;  // the wave's 32 rows of the workgroup's, and its keys of each block
   const int lr = lane & 15, lq = lane >> 4;
   const int p0 = first_pos(p.pos0, b, p.T, p.cap);
 
   const int row0 = rb * PR;
   const int t_last = min((row0 + PR - 1) / g, p.T - 1);
-  const int k_hi = min(p0 + t_last + 1, p.split_len);  // keys of this workgroup: [0, k_hi)
-  const int k_free = min(p0 + row0 / g + 1, k_hi);      // keys below this are visible to every row
+  const int k_lo = split * p.split_len;
+  const int k_hi = min(p0 + t_last + 1, k_lo + p.split_len);  // keys of this workgroup: [k_lo, k_hi)
+  const int k_free = min(p0 + row0 / g + 1, k_hi);             // keys below this are visible to every row
+  const int nblk = k_hi > k_lo ? (k_hi - k_lo + KB - 1) / KB : 0;
 
-  // the wave's two 16-row tiles; rows past the end compute on q = 0 and are not stored
-  int t[2], hq[2], kmax[2];
-  bool row_ok[2];
-  bf16x8 qf[2][NS];
+  // the wave's two 16-row tiles; rows past the end compute on q = 0 and are not stored.  The last QL
+  // k-steps of q are kept in LDS (both waves of a row group read one copy)
+  auto q_lds = [&](int rt, int s) {
+    return reinterpret_cast<bf16x8*>(smem + 2 * (KSTAGE + VSTAGE) + kMl) +
+           ((rg * 2 + rt) * QL + s - (NS - QL)) * 64 + lane;
+  };
+  int kmax[2];
+  bf16x8 qf[2][NS - QL];
 #pragma unroll
   for (int rt = 0; rt < 2; ++rt) {
-    const int r = row0 + 32 * wave + 16 * rt + lr;
-    row_ok[rt] = r < n_rows;
-    t[rt] = row_ok[rt] ? r / g : p.T - 1;
-    hq[rt] = hkv * g + (row_ok[rt] ? r % g : 0);
-    kmax[rt] = p0 + t[rt];
-    const uint16_t* qrow = p.q + ((static_cast<int64_t>(b) * p.T + t[rt]) * p.Hq + hq[rt]) * D;
+    const int r = row0 + 32 * rg + 16 * rt + lr;
+    const bool ok = r < n_rows;
+    const int t = ok ? r / g : p.T - 1, hq = hkv * g + (ok ? r % g : 0);
+    kmax[rt] = p0 + t;
+    const uint16_t* qrow = p.q + ((static_cast<int64_t>(b) * p.T + t) * p.Hq + hq) * D;
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
       const u32x4 v = *reinterpret_cast<const u32x4*>(qrow + 32 * s + 8 * lq);
-      qf[rt][s] = __builtin_bit_cast(bf16x8, row_ok[rt] ? v : u32x4{0u, 0u, 0u, 0u});
+      const bf16x8 f = __builtin_bit_cast(bf16x8, ok ? v : u32x4{0u, 0u, 0u, 0u});
+      if (s < NS - QL) qf[rt][s] = f;
+      else if (kh == 0) *q_lds(rt, s) = f;
     }
   }
 
-  const uint16_t* kc_head = p.kc + (static_cast<int64_t>(b) * p.Hkv + hkv) * p.cap * D;
-  const uint16_t* vc_head = p.vc + (static_cast<int64_t>(b) * p.Hkv + hkv) * p.cap * D;
-  // K block kb -> stage st: thread tid's load i fills physical granule i * 256 + tid, which is row
-  // i * KR + tid / KG, granule (tid % KG) ^ (row & 7) of the block (the swizzle does not depend on i)
-  constexpr int KR = 256 / KG;
-  const int k_row0 = tid / KG;
-  const int k_off = k_row0 * D + (((tid % KG) ^ (k_row0 & 7)) * 8);
+  // K and V blocks are read through descriptors that end at the range's last
+  // key, so the lane offsets are constants and keys past the range (masked
+  // below) read as zeros
+  const unsigned char* kc_head =
+      reinterpret_cast<const unsigned char*>(p.kc + (static_cast<int64_t>(b) * p.Hkv + hkv) * p.cap * D);
+  const unsigned char* vc_head =
+      reinterpret_cast<const unsigned char*>(p.vc + (static_cast<int64_t>(b) * p.Hkv + hkv) * p.cap * D);
+  auto block_bytes = [&](int kb) { return min(k_hi - kb, KB) * (D * 2); };
+  // K block -> stage st: thread tid's load i fills physical granule i * NT + tid, which is row
+  // i * KR + tid / KROW, granule (tid % KROW) ^ (row & 7) of the block (the swizzle does not depend on i)
+  constexpr int KR = NT / KROW;
+  static_assert(KR % 8 == 0, "the swizzle of a granule must not depend on the load");
+  const int k_row0 = tid / KROW;
+  const uint32_t k_off = k_row0 * (D * 2) + (((tid % KROW) ^ (k_row0 & 7)) * 16);
   // LDS address of the wave's 1 KB slice of load 0 in stage 0
   const uint32_t k_lds = __builtin_amdgcn_readfirstlane(
       static_cast<uint32_t>(reinterpret_cast<uintptr_t>(smem)) + wave * 1024);
-  // keys past the range re-read the last one (in bounds; they are masked)
-  auto k_dma = [&](int kb, int st, int i) {
-    const int key = min(kb + i * KR + k_row0, k_hi - 1);
-    lds_dma16(kc_head + static_cast<int64_t>(key) * D + (k_off - k_row0 * D), k_lds + st * KSTAGE + i * 4096);
+  auto k_dma = [&](int kb, int bytes, int st, int i) {  // the block's bytes from load i's first row on
+    constexpr int kLoad = KR * D * 2;
+    lds_dma16(buf_words(kc_head + static_cast<int64_t>(kb) * (D * 2) + i * kLoad, max(bytes - i * kLoad, 0)), k_off,
+              k_lds + st * KSTAGE + i * (NT * 16));
   };
-  // V block kb -> registers: pair i is key quad tid % 16 (4 rows) x d octet i * 16 + tid / 16
+  // V block -> registers: pair i is key quad tid % 16 (4 rows) x d octet i * NT / 16 + tid / 16
   const int v_kq = tid % (KB / 4), v_dq = tid / (KB / 4);
+  const uint32_t v_off = 4 * v_kq * (D * 2) + v_dq * 16;
   u32x4 vr[VPAIRS][4];
-  auto v_load = [&](int kb, int i, int e) {
-    const int key = min(kb + 4 * v_kq + e, k_hi - 1);
-    vr[i][e] = *reinterpret_cast<const u32x4*>(vc_head + static_cast<int64_t>(key) * D + (v_dq + i * 16) * 8);
+  auto v_load = [&](__amdgpu_buffer_rsrc_t rsrc, int i, int e) {
+    vr[i][e] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, v_off + e * (D * 2) + i * NT, 0, 0);
   };
   // registers -> Vt stage st: for each of the octet's 8 d, the quad's 4 keys as one 8-byte write
   const int v_pos = 32 * (v_kq >> 3) + 8 * (v_kq & 3) + 4 * ((v_kq >> 2) & 1);
   const int v_gran = v_pos >> 3, v_half = v_pos & 7;  // the position's granule and offset in it
-  auto v_store = [&](int st, int i, int m) {  // d rows 8 (v_dq + 16 i) + 2m, + 2m + 1 (d & 7 = 2m, 2m + 1)
-    uint16_t* Vt = reinterpret_cast<uint16_t*>(smem + 2 * KSTAGE + st * VSTAGE) + (8 * (v_dq + i * 16)) * VTP + v_half;
+  // byte offset of d row 8 v_dq's piece; row + c is at (this ^ (c << 4)) + c rows (a row's 128 bytes are aligned)
+  const int v_at = 2 * KSTAGE + 8 * v_dq * (VTP * 2) + 16 * v_gran + 2 * v_half;
+  auto v_store = [&](int st, int i, int m) {  // d rows 8 (v_dq + i NT / 16) + 2m, + 2m + 1 (d & 7 = 2m, 2m + 1)
+    const int at = v_at + st * VSTAGE + i * (NT / 2) * (VTP * 2);
     const uint32_t k0 = vr[i][0][m], k1 = vr[i][1][m], k2 = vr[i][2][m], k3 = vr[i][3][m];
-    const u32x2 even = {(k0 & 0xffffu) | (k1 << 16), (k2 & 0xffffu) | (k3 << 16)};
-    const u32x2 odd = {(k0 >> 16) | (k1 & 0xffff0000u), (k2 >> 16) | (k3 & 0xffff0000u)};
-    *reinterpret_cast<u32x2*>(Vt + (2 * m) * VTP + ((v_gran ^ (2 * m)) << 3)) = even;
-    *reinterpret_cast<u32x2*>(Vt + (2 * m + 1) * VTP + ((v_gran ^ (2 * m + 1)) << 3)) = odd;
+    // byte permutes: the low (0x05040100) and the high (0x07060302) halves of two keys' words
+    const u32x2 even = {__builtin_amdgcn_perm(k1, k0, 0x05040100u), __builtin_amdgcn_perm(k3, k2, 0x05040100u)};
+    const u32x2 odd = {__builtin_amdgcn_perm(k1, k0, 0x07060302u), __builtin_amdgcn_perm(k3, k2, 0x07060302u)};
+    *reinterpret_cast<u32x2*>(smem + (at ^ (2 * m << 4)) + (2 * m) * (VTP * 2)) = even;
+    *reinterpret_cast<u32x2*>(smem + (at ^ ((2 * m + 1) << 4)) + (2 * m + 1) * (VTP * 2)) = odd;
   };
 
-  float m[2] = {-INFINITY, -INFINITY}, l[2] = {0.0f, 0.0f};
+  // a wave may see no key of a row in its range: the running max starts at a
+  // finite value, so that exp2 of a masked score is 0 and not exp2(-inf + inf)
+  float m[2] = {-FLT_MAX, -FLT_MAX}, l[2] = {0.0f, 0.0f};
   f32x4 o[2][NJ];
 #pragma unroll
   for (int rt = 0; rt < 2; ++rt)
@@ -630,72 +694,87 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(const AttnParams p) {
   // = 8 (s >> 1) + 4 ((s & 1) ^ x2) + (q ^ x01) with x = r & 7: one base for even s, one for odd,
   // each plus 64 (s & ~1) bytes
   const int x2 = (lr >> 2) & 1, y01 = lq ^ (lr & 3);
-  const int kfe = lr * (D * 2) + (4 * x2 + y01) * 16, kfo = lr * (D * 2) + (4 * (x2 ^ 1) + y01) * 16;
+  const int kf0 = 16 * KTW * kh * (D * 2) + lr * (D * 2);
+  const int kfe = kf0 + (4 * x2 + y01) * 16, kfo = kf0 + (4 * (x2 ^ 1) + y01) * 16;
   // V^T fragment (j, ks) of lane (r, q): d row 16 j + r, positions 32 ks + 8q .., granule (4 ks + q) ^ (r & 7)
-  const int vfo0 = lr * (VTP * 2) + (4 * x2 + y01) * 16, vfo1 = lr * (VTP * 2) + (4 * (x2 ^ 1) + y01) * 16;
+  const int vfo0 = lr * (VTP * 2) + (4 * (x2 ^ (KG == 2 ? kh : 0)) + y01) * 16;
+  const int vfo1 = lr * (VTP * 2) + (4 * (x2 ^ 1) + y01) * 16;
 
-  const int nblk = (k_hi + KB - 1) / KB;  // >= 1: k_hi > p0 + row0 / g >= 0
+  // Every wave's LDS writes and direct loads are visible to the others.  The 4 VPAIRS loads of V issued after
+  // the direct loads may stay in flight (they go to this thread's registers).
+  auto publish = [&]() {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(4 * VPAIRS) : "memory");
+  };
+  if (nblk > 0) {
+    const int nb = block_bytes(k_lo);
+    const int k1 = nblk > 1 ? k_lo + KB : k_lo;
+    const __amdgpu_buffer_rsrc_t vrs = buf_rsrc(vc_head + static_cast<int64_t>(k_lo) * (D * 2), nb);
+    const __amdgpu_buffer_rsrc_t vrs1 = buf_rsrc(vc_head + static_cast<int64_t>(k1) * (D * 2), block_bytes(k1));
 #pragma unroll
-  for (int i = 0; i < KDMA; ++i) k_dma(0, 0, i);
+    for (int i = 0; i < KDMA; ++i) k_dma(k_lo, nb, 0, i);
 #pragma unroll
-  for (int i = 0; i < VPAIRS; ++i) {
+    for (int i = 0; i < VPAIRS; ++i) {
 #pragma unroll
-    for (int e = 0; e < 4; ++e) v_load(0, i, e);
+      for (int e = 0; e < 4; ++e) v_load(vrs, i, e);
+    }
 #pragma unroll
-    for (int m = 0; m < 4; ++m) v_store(0, i, m);
+    for (int i = 0; i < VPAIRS; ++i) {
+#pragma unroll
+      for (int m4 = 0; m4 < 4; ++m4) v_store(0, i, m4);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v_load(vrs1, i, e);
+    }
   }
   for (int blk = 0; blk < nblk; ++blk) {
-    const int kb = KB * blk, st = blk & 1;
-    __builtin_amdgcn_s_waitcnt(0);  // this thread's direct loads of block blk have landed
-    __syncthreads();                // everyone's have, Vt[st] is written, stage st ^ 1 is free
-    // the next block's K and V go in while this one computes: one K load and one V load per k-step of
-    // S^T, V stored (transposed) during O^T; the last block re-reads itself into the free stage (never
-    // read) so that no load sits behind a branch
-    const int kb_next = blk + 1 < nblk ? kb + KB : kb;
+    const int kb = k_lo + KB * blk, st = blk & 1;
+    publish();  // block blk is in LDS, stage st ^ 1 is free
+    // K of the next block goes in during S^T; its V (in registers since the last iteration) is stored,
+    // transposed, during O^T, and the registers take the block after it.  Past the end the loads re-read the
+    // last block (never used), so that none sits behind a branch.
+    const int kb1 = blk + 1 < nblk ? kb + KB : kb, kb2 = blk + 2 < nblk ? kb + 2 * KB : kb1;
+    const int nb1 = block_bytes(kb1);
+    const __amdgpu_buffer_rsrc_t vrs = buf_rsrc(vc_head + static_cast<int64_t>(kb2) * (D * 2), block_bytes(kb2));
 
     // S^T = K Q^T: lane (r, q) holds keys 16 kt + 4q + i of row r, for both row tiles
     const unsigned char* Ks = smem + st * KSTAGE;
     auto k_frag = [&](int s, int kt) {
       return *reinterpret_cast<const bf16x8*>(Ks + ((s & 1) ? kfo : kfe) + kt * 16 * (D * 2) + (s & ~1) * 64);
     };
-    f32x4 sc[2][4];
+    f32x4 sc[2][KTW];
 #pragma unroll
-    for (int kt = 0; kt < 4; ++kt) sc[0][kt] = sc[1][kt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    bf16x8 kf[2][4];  // the fragments of k-step s, and those of s + 1 in flight
+    for (int kt = 0; kt < KTW; ++kt) sc[0][kt] = sc[1][kt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    // fragments f = (k-step f / KTW, tile f % KTW), KPF of them in flight
+    constexpr int KPF = KG == 2 ? 3 : 4;
+    bf16x8 kf[KPF];
 #pragma unroll
-    for (int kt = 0; kt < 4; ++kt) kf[0][kt] = k_frag(0, kt);
+    for (int f = 0; f < KPF; ++f) kf[f] = k_frag(f / KTW, f % KTW);
 #pragma unroll
-    for (int s = 0; s < NS; ++s) {
-      if (s + 1 < NS) {
-#pragma unroll
-        for (int kt = 0; kt < 4; ++kt) kf[(s + 1) & 1][kt] = k_frag(s + 1, kt);
-      }
-      static_assert(KDMA == NS, "one K load per k-step");
-      k_dma(kb_next, st ^ 1, s);
-      if (s < 4 * VPAIRS) v_load(kb_next, s / 4, s % 4);
-#pragma unroll
-      for (int kt = 0; kt < 4; ++kt) {
-        sc[0][kt] = mfma16(kf[s & 1][kt], qf[0][s], sc[0][kt]);
-        sc[1][kt] = mfma16(kf[s & 1][kt], qf[1][s], sc[1][kt]);
-      }
+    for (int f = 0; f < NS * KTW; ++f) {
+      const int s = f / KTW, kt = f % KTW;
+      const bf16x8 a = kf[f % KPF];
+      if (f + KPF < NS * KTW) kf[f % KPF] = k_frag((f + KPF) / KTW, (f + KPF) % KTW);
+      if (kt == 0 && s < KDMA) k_dma(kb1, nb1, st ^ 1, s);
+      const bool in_regs = s < NS - QL;
+      sc[0][kt] = mfma16(a, in_regs ? qf[0][in_regs ? s : 0] : *q_lds(0, s), sc[0][kt]);
+      sc[1][kt] = mfma16(a, in_regs ? qf[1][in_regs ? s : 0] : *q_lds(1, s), sc[1][kt]);
     }
-    // issue order: k-step s + 1's four fragment reads ahead of k-step s's eight products
-    __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
+    // issue order: fragment f + KPF read ahead of fragment f's two products
+    __builtin_amdgcn_sched_group_barrier(0x100, KPF, 0);
 #pragma unroll
-    for (int s = 0; s < NS; ++s) {
-      if (s + 1 < NS) __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
-      if (s < 4 * VPAIRS) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(0x008, 8, 0);
+    for (int f = 0; f < NS * KTW; ++f) {
+      if (f + KPF < NS * KTW) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+      if (f % KTW == 0 && f / KTW >= NS - QL) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);  // q
+      __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
     }
 
     if (kb + KB > k_free) {
 #pragma unroll
       for (int rt = 0; rt < 2; ++rt)
 #pragma unroll
-        for (int kt = 0; kt < 4; ++kt)
+        for (int kt = 0; kt < KTW; ++kt)
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
-            const int key = kb + 16 * kt + 4 * lq + i;
+            const int key = kb + 16 * (KTW * kh + kt) + 4 * lq + i;
             if (!(key <= kmax[rt] && key < k_hi)) sc[rt][kt][i] = -INFINITY;
           }
     }
@@ -705,7 +784,7 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(const AttnParams p) {
     for (int rt = 0; rt < 2; ++rt) {
       float x = -INFINITY;
 #pragma unroll
-      for (int kt = 0; kt < 4; ++kt)
+      for (int kt = 0; kt < KTW; ++kt)
 #pragma unroll
         for (int i = 0; i < 4; ++i) x = fmaxf(x, sc[rt][kt][i]);
       mb[rt] = rows_max(x) * p.scale_log2;
@@ -724,12 +803,12 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(const AttnParams p) {
     }
     // P = exp2(s * scale - m) as the B operand of O^T += V^T P^T: k-slots 8q .. 8q+3 are keys
     // 32 ks + 4q + (0..3) (accumulator tile 2 ks), 8q+4 .. 8q+7 are keys 32 ks + 16 + 4q + (0..3)
-    bf16x8 pb[2][2];
+    bf16x8 pb[2][KSW];
 #pragma unroll
     for (int rt = 0; rt < 2; ++rt) {
       float ps = 0.0f;
 #pragma unroll
-      for (int kt = 0; kt < 4; ++kt)
+      for (int kt = 0; kt < KTW; ++kt)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           sc[rt][kt][i] = __builtin_amdgcn_exp2f(fmaf(sc[rt][kt][i], p.scale_log2, -m[rt]));
@@ -737,7 +816,7 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(const AttnParams p) {
         }
       l[rt] += ps;
 #pragma unroll
-      for (int ks = 0; ks < 2; ++ks)
+      for (int ks = 0; ks < KSW; ++ks)
         pb[rt][ks] = __builtin_bit_cast(
             bf16x8, u32x4{pk_bf16(sc[rt][2 * ks][0], sc[rt][2 * ks][1]), pk_bf16(sc[rt][2 * ks][2], sc[rt][2 * ks][3]),
                           pk_bf16(sc[rt][2 * ks + 1][0], sc[rt][2 * ks + 1][1]),
@@ -746,8 +825,8 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(const AttnParams p) {
 
     // O^T += V^T P^T
     const unsigned char* Vt = smem + 2 * KSTAGE + st * VSTAGE;
-    constexpr int NF = 2 * NJ;  // V^T fragments per block: (ks, j) = (f / NJ, f % NJ)
-    constexpr int VPF = 4;      // fragments in flight
+    constexpr int NF = KSW * NJ;  // V^T fragments per block: (ks, j) = (f / NJ, f % NJ)
+    constexpr int VPF = 4;        // fragments in flight
     auto v_frag = [&](int f) {
       return *reinterpret_cast<const bf16x8*>(Vt + (f / NJ ? vfo1 : vfo0) + (f % NJ) * 16 * (VTP * 2));
     };
@@ -762,7 +841,14 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(const AttnParams p) {
       o[0][j] = mfma16(a, pb[0][ks], o[0][j]);
       o[1][j] = mfma16(a, pb[1][ks], o[1][j]);
       // the next block's V into the free stage
-      if (f % 2 == 1 && f / 2 < 4 * VPAIRS) v_store(st ^ 1, f / 8, (f / 2) % 4);
+      constexpr int VST = NF / (4 * VPAIRS);  // fragments per transposed store
+      if (f % VST == VST - 1) {
+        v_store(st ^ 1, f / VST / 4, (f / VST) % 4);
+        if ((f / VST) % 4 == 3) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v_load(vrs, f / VST / 4, e);
+        }
+      }
     }
     // issue order: fragment f + VPF read ahead of fragment f's two products
     __builtin_amdgcn_sched_group_barrier(0x100, VPF, 1);
@@ -771,48 +857,120 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(const AttnParams p) {
       if (f + VPF < NF) __builtin_amdgcn_sched_group_barrier(0x100, 1, 1);
       __builtin_amdgcn_sched_group_barrier(0x008, 2, 1);
     }
-
   }
 
+  __builtin_amdgcn_s_waitcnt(0);  // no direct load may land in LDS after this
+  float lt[2] = {rows_sum(l[0]), rows_sum(l[1])};
+  // row tile rt's state (lane (r, q): O[row r][16 j + 4 q + i]) to the output, or to the split's partials
+  auto store_tile = [&](auto rtc) {
+    constexpr int rt = decltype(rtc)::value;
+    const int r = row0 + 32 * rg + 16 * rt + lr;
+    if (r >= n_rows) return;
+    if (p.n_split == 1) {
+      const float inv_l = lt[rt] > 0.0f ? 1.0f / lt[rt] : 0.0f;
 #pragma unroll
-  for (int rt = 0; rt < 2; ++rt) {
-    const float lt = rows_sum(l[rt]);
-    if (!row_ok[rt]) continue;
-    const float inv_l = lt > 0.0f ? 1.0f / lt : 0.0f;
+      for (int j = 0; j < NJ; ++j) store_out4<D>(p, b, r / g, hkv * g + r % g, 16 * j + 4 * lq, o[rt][j], inv_l);
+      return;
+    }
+    const int64_t pr = part_row(p, b, hkv, r) + split;
+    const int64_t n_part = static_cast<int64_t>(p.B) * p.Hkv * p.rows_pad * p.n_split;
+    if (lq == 0) {
+      p.part[n_part * D + pr] = m[rt];
+      p.part[n_part * (D + 1) + pr] = lt[rt];
+    }
+    if (nblk == 0) return;  // the combine does not read the O of a range without keys (l = 0)
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) store_out4<D>(p, b, t[rt], hq[rt], 16 * j + 4 * lq, o[rt][j], inv_l);
+    for (int j = 0; j < NJ; ++j) *reinterpret_cast<f32x4*>(p.part + pr * D + 16 * j + 4 * lq) = o[rt][j];
+  };
+  if constexpr (KG == 1) {
+    store_tile(std::integral_constant<int, 0>{});
+    store_tile(std::integral_constant<int, 1>{});
+  } else {
+    // the two waves of a row group merge: wave kh finishes row tile kh, and
+    // hands its state of the other tile over in LDS (the K / V stages are free)
+    float* xo = reinterpret_cast<float*>(smem);  // [8 waves][NJ][64 lanes][4]
+    float* xml = xo + 8 * NJ * 256;              // [8 waves][2][64 lanes]
+    static_assert(8 * NJ * 256 * 4 <= 2 * (KSTAGE + VSTAGE), "the exchange must fit in the stages");
+    __syncthreads();
+    auto hand_over = [&](auto rtc) {
+      constexpr int rt = decltype(rtc)::value;
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) *reinterpret_cast<f32x4*>(xo + ((wave * NJ + j) * 64 + lane) * 4) = o[rt][j];
+      xml[wave * 128 + lane] = m[rt];
+      xml[wave * 128 + 64 + lane] = lt[rt];
+    };
+    auto finish = [&](auto rtc) {
+      constexpr int rt = decltype(rtc)::value;
+      const int w = wave ^ 4;
+      const float m2 = xml[w * 128 + lane], l2 = xml[w * 128 + 64 + lane];
+      const float mm = fmaxf(m[rt], m2);
+      const float a1 = __builtin_amdgcn_exp2f(m[rt] - mm), a2 = __builtin_amdgcn_exp2f(m2 - mm);
+      m[rt] = mm;
+      lt[rt] = a1 * lt[rt] + a2 * l2;
+#pragma unroll
+      for (int j = 0; j < NJ; ++j)
+        o[rt][j] = a1 * o[rt][j] + a2 * *reinterpret_cast<const f32x4*>(xo + ((w * NJ + j) * 64 + lane) * 4);
+      store_tile(rtc);
+    };
+    if (kh == 0) hand_over(std::integral_constant<int, 1>{});
+    else hand_over(std::integral_constant<int, 0>{});
+    __syncthreads();
+    if (kh == 0) finish(std::integral_constant<int, 0>{});
+    else finish(std::integral_constant<int, 1>{});
   }
 }
 
 // One wave per (row, kv-head, batch row): the split partials of a row merged.
+// A range without keys of the row (l = 0) may have left its O unwritten: it is
+// skipped, its loads read the row's first range with keys instead.
+// Lane s takes range s's m and l (64 ranges a pass), and eight ranges' O are
+// in flight at a time.
 template <int D>
 __global__ __launch_bounds__(256) void attn_combine_kernel(const AttnParams p) {
   const int lane = threadIdx.x & 63;
   const int g = p.Hq / p.Hkv;
   const int n_rows = p.T * g;
-  const int64_t item = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
+  const int64_t item =
+      static_cast<int64_t>(blockIdx.x) * 4 + __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
   if (item >= static_cast<int64_t>(p.B) * p.Hkv * n_rows) return;
   const int r = static_cast<int>(item % n_rows);
   const int hkv = static_cast<int>((item / n_rows) % p.Hkv);
   const int b = static_cast<int>(item / (static_cast<int64_t>(n_rows) * p.Hkv));
   const int64_t n_part = static_cast<int64_t>(p.B) * p.Hkv * p.rows_pad * p.n_split;
-  const float* ml = p.part + n_part * D;
   const int64_t pr = part_row(p, b, hkv, r);
-  float ms = -INFINITY;
-  for (int s = 0; s < p.n_split; ++s) ms = fmaxf(ms, ml[pr + s]);
-  const float m_use = ms == -INFINITY ? 0.0f : ms;
-  constexpr int EPL = D / 64;
-  f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-  float lsum = 0.0f;
-  for (int s = 0; s < p.n_split; ++s) {
-    const float w = __builtin_amdgcn_exp2f(ml[pr + s] - m_use);
-    lsum += w * ml[n_part + pr + s];
-    const float* po = p.part + (pr + s) * D + EPL * lane;
-    if constexpr (EPL == 4) {
-      acc += w * *reinterpret_cast<const f32x4*>(po);
-    } else {
-      acc[0] += w * po[0];
-      acc[1] += w * po[1];
+  const float* pm = p.part + n_part * D + pr;
+  const float* pl = p.part + n_part * (D + 1) + pr;
+  constexpr int EPL = D / 64, NB = 8;
+  typedef float vec __attribute__((ext_vector_type(EPL)));
+  vec acc = {};
+  float m = -FLT_MAX, lsum = 0.0f;
+  for (int s0 = 0; s0 < p.n_split; s0 += 64) {
+    const int n = min(64, p.n_split - s0);
+    const float ls = lane < n ? pl[s0 + lane] : 0.0f;
+    const float ms = lane < n && ls != 0.0f ? pm[s0 + lane] : -FLT_MAX;
+    const uint64_t has = __builtin_amdgcn_ballot_w64(ls != 0.0f);
+    if (has == 0) continue;
+    const int first = __builtin_ctzll(has);
+    const float m_new = fmaxf(m, wave_max(ms));
+    const float keep = __builtin_amdgcn_exp2f(m - m_new);
+    m = m_new;
+    const float w = __builtin_amdgcn_exp2f(ms - m);  // the lane's range
+    acc *= keep;
+    lsum = lsum * keep + wave_sum(ls != 0.0f ? w * ls : 0.0f);
+    for (int s = 0; s < n; s += NB) {
+      vec v[NB];
+#pragma unroll
+      for (int i = 0; i < NB; ++i) {
+        const int si = min(s + i, n - 1);
+        const int src = (has >> si) & 1 ? si : first;
+        v[i] = *reinterpret_cast<const vec*>(p.part + (pr + s0 + src) * D + EPL * lane);
+      }
+#pragma unroll
+      for (int i = 0; i < NB; ++i) {
+        const int si = min(s + i, n - 1);
+        const float wi = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(w), si));
+        if (s + i < n && ((has >> si) & 1)) acc += wi * v[i];  // wave-uniform
+      }
     }
   }
   const float inv_l = lsum > 0.0f ? 1.0f / lsum : 0.0f;
@@ -1079,16 +1237,14 @@ extern "C" int gdn_attn_fwd(const void* q, const void* qg, int64_t qg_ld, const 
   p.rows_pad = static_cast<int>(rows_pad);
   p.scale_log2 = scale * kLog2e;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  if (n_split == 1 && T * (Hq / Hkv) >= kPrefillRows) {
+  if (T * (Hq / Hkv) >= kPrefillRows) {
     const int64_t n_prb = (T * (Hq / Hkv) + PR - 1) / PR;
     if (Hkv * n_prb > INT32_MAX) return fail(GDN_ERR_UNSUPPORTED, "gdn_attn_fwd: problem too large");
-    const dim3 pgrid(static_cast<unsigned>(Hkv * n_prb), 1, static_cast<unsigned>(B));
-    if (D == 256) hipLaunchKernelGGL(attn_prefill_kernel<256>, pgrid, dim3(256), 0, st, p);
-    else hipLaunchKernelGGL(attn_prefill_kernel<128>, pgrid, dim3(256), 0, st, p);
-    return gdn_host::check_launch("gdn_attn_fwd/prefill");
-  }
-  const dim3 grid(static_cast<unsigned>(n_split), static_cast<unsigned>(Hkv * n_rb), static_cast<unsigned>(B));
-  if (D == 256) {
+    const dim3 pgrid(static_cast<unsigned>(Hkv * n_prb), static_cast<unsigned>(n_split), static_cast<unsigned>(B));
+    if (D == 256) hipLaunchKernelGGL((attn_prefill_kernel<256, 2>), pgrid, dim3(512), 0, st, p);
+    else hipLaunchKernelGGL((attn_prefill_kernel<128, 1>), pgrid, dim3(256), 0, st, p);
+  } else if (const dim3 grid(static_cast<unsigned>(n_split), static_cast<unsigned>(Hkv * n_rb), static_cast<unsigned>(B));
+             D == 256) {
     if (rt == 4) hipLaunchKernelGGL((attn_fwd_kernel<256, 4>), grid, dim3(256), 0, st, p);
     else hipLaunchKernelGGL((attn_fwd_kernel<256, 1>), grid, dim3(256), 0, st, p);
   } else {

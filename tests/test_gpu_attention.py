@@ -167,6 +167,12 @@ CASES = {
     "verify_t4_split_d128": (4, 4, [3, 100, 257, 0], 3, True, (16, 4, 128)),
     "rt4_split_d128": (2, 8, [5, 300], 3, False, (16, 4, 128)),
     "prefill_short_d128": (2, 40, [0, 17], 1, True, (16, 4, 128)),
+    # 128-row tiles with keys split over workgroups: ranges without keys (row 0), one block
+    # per range, a last tile of 8 rows; and more ranges than the combine takes in one pass
+    "prefill_split_empty": (2, 130, [0, 700], 5, True),
+    "prefill_split_blocks": (1, 128, [2000], 33, True),
+    "prefill_split_d128": (1, 300, [333], 3, False, (16, 4, 128)),
+    "decode_split_70": (1, 1, [4500], 70, True),
 }
 
 
