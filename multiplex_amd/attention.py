@@ -425,16 +425,31 @@ class Attention(torch.nn.Module):
         self.k_norm.weight.copy_(k_norm)
 
     def _splits(self, B: int, T: int, L: int) -> int:
-        """Key ranges per row for decode and draft verify: about one
-        workgroup per CU (measured best: one 68 KB-LDS workgroup per CU
-        streams the cache faster than two), ranges of at least 512 keys."""
+        """Key ranges per row, where the rows alone leave CUs idle (measured
+        at 4 kv-heads of 256, us with one range and with the rule's).
+
+        At least 512 rows (tokens x heads of a group) a kv-head: the 128-row
+        tiles' workgroups, one per CU, times the ranges fit the CUs, each at
+        least 256 keys of the prefix (512 tokens over 4096: 129 -> 61; 128
+        over 8192: 216 -> 43; 1024 over none stays whole: 42, two ranges 47).
+        Up to 16 rows (decode, draft verify): about one workgroup per CU, more
+        than 64 keys (one token over 1024: 36 -> 14, over 256: 13.1 -> 11.6,
+        over 128: 9.9, two ranges 11.0).  Between: 64-row tiles, two workgroups per CU; at least
+        128 keys up to one workgroup per CU and 256 beyond (8 tokens over
+        16384: 853 -> 35; 32 over 1024: 60 -> 20; 64 over 8192: 430 -> 45).
+        """
         if self.n_split is not None:
             return self.n_split
-        if T * (self.Hq // self.Hkv) > 16:
-            return 1
         if self._cus is None:
             self._cus = torch.cuda.get_device_properties(self.qkv_proj.device).multi_processor_count
-        return int(max(1, min(round(self._cus / (B * self.Hkv)), L // 512)))
+        rows = T * (self.Hq // self.Hkv)
+        if rows >= 512:
+            n = B * self.Hkv * -(-rows // 128)
+            return max(1, min(self._cus // n, (L - T) // 256))
+        if rows <= 16:
+            return max(1, min(round(self._cus / (B * self.Hkv)), L // 64 - 1))
+        n = B * self.Hkv * -(-rows // 64)
+        return max(1, min(self._cus // n, L // 128), min(2 * self._cus // n, L // 256))
 
     def forward(self, x: torch.Tensor, cache: KVCache) -> torch.Tensor:
         B, T, _ = x.shape
