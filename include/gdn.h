@@ -411,12 +411,18 @@ size_t gdn_linear_decode_workspace_bytes(int64_t M, int64_t N, int64_t K);
  * slices of one output tile are summed in slice order, so results do not
  * depend on scheduling.  With the norm fused it is faster than the separate
  * norm plus a library GEMM up to 16 rows, and slower beyond (at hidden 2048,
- * graph-replayed); without the norm the library GEMM is faster.
+ * graph-replayed); without the norm the library GEMM is faster beyond 16
+ * rows, and up to 16 (more than 2048 columns) gdn_linear_rows16's kernel runs.
  */
 int gdn_linear_decode(const void* x, int64_t ldx, const void* gate, int64_t ldg, const void* norm_w,
                       int norm_w_dtype, float eps, int64_t head_dim, const void* W, void* out,
                       int64_t ldo, int64_t M, int64_t N, int64_t K, void* workspace,
                       size_t workspace_bytes, void* stream);
+
+/* out[M, N] = x[M, K] W[N, K]^T as gdn_linear_decode without a gate, for
+ * 1 <= M <= 16 and without a workspace: one workgroup per output tile. */
+int gdn_linear_rows16(const void* x, int64_t ldx, const void* W, void* out, int64_t ldo, int64_t M,
+                      int64_t N, int64_t K, void* stream);
 
 #ifdef __cplusplus
 }

@@ -50,6 +50,7 @@ EXPORTS = (
     "gdn_rms_norm",
     "gdn_silu_mul",
     "gdn_linear_decode_workspace_bytes",
+    "gdn_linear_rows16",
     "gdn_linear_decode",
 )
 
@@ -171,6 +172,7 @@ _SIGNATURES = {
     "gdn_rms_norm": (c_int, [_P, _P, _P, _P, c_int, _P, _I64, _I64, _I64, c_float, _P]),
     "gdn_silu_mul": (c_int, [_P, _P, _I64, _I64, _P]),
     "gdn_linear_decode_workspace_bytes": (c_size_t, [_I64, _I64, _I64]),
+    "gdn_linear_rows16": (c_int, [_P, _I64, _P, _P, _I64, _I64, _I64, _I64, _P]),
     "gdn_linear_decode": (
         c_int,
         [_P, _I64, _P, _I64, _P, c_int, c_float, _I64, _P, _P, _I64, _I64, _I64, _I64, _P, c_size_t, _P],

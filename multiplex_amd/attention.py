@@ -14,7 +14,7 @@ call shapes:
                  ``offset`` / ``size()`` / ``trim(n)`` / ``state`` /
                  ``filter`` / ``extract`` / ``merge`` as the drafter uses them
   Attention      Qwen3.5 gated attention: one GEMM for q|gate, k and v
-                 (hipBLASLt through torch), then ``gdn_attn_qk`` (q/k RMSNorm,
+                 (:func:`multiplex_amd.linear.linear`), then ``gdn_attn_qk`` (q/k RMSNorm,
                  partial rotary embedding, cache append) and ``gdn_attn_fwd``
                  (GQA flash attention on bf16 MFMA with the sigmoid gate
                  fused), then o_proj
@@ -37,6 +37,7 @@ import torch
 
 from . import _lib
 from .gated_delta import _dtype_code, _ptr, _require_device, _stream
+from .linear import linear
 
 __all__ = [
     "AttentionArgs",
@@ -454,7 +455,7 @@ class Attention(torch.nn.Module):
     def forward(self, x: torch.Tensor, cache: KVCache) -> torch.Tensor:
         B, T, _ = x.shape
         Hq, Hkv, D = self.Hq, self.Hkv, self.D
-        qkv = torch.nn.functional.linear(x, self.qkv_proj)
+        qkv = linear(x, self.qkv_proj)
         qg = qkv[..., : 2 * Hq * D]
         k = qkv[..., 2 * Hq * D : (2 * Hq + Hkv) * D]
         v = qkv[..., (2 * Hq + Hkv) * D :]
@@ -465,7 +466,7 @@ class Attention(torch.nn.Module):
         o = attn_fwd(q, cache.keys, cache.values, cache.pos0, L, gate=qg, scale=self.scale,
                      n_split=self._splits(B, T, L))
         cache.advance(T)
-        return torch.nn.functional.linear(o.view(B, T, Hq * D), self.o_proj)
+        return linear(o.view(B, T, Hq * D), self.o_proj)
 
 
 class MLP(torch.nn.Module):
@@ -482,7 +483,7 @@ class MLP(torch.nn.Module):
         self.down_proj.copy_(down_proj.to(self.down_proj))
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        return torch.nn.functional.linear(silu_mul(torch.nn.functional.linear(x, self.gate_up_proj)), self.down_proj)
+        return linear(silu_mul(linear(x, self.gate_up_proj)), self.down_proj)
 
 
 class DecoderLayer(torch.nn.Module):
@@ -542,7 +543,7 @@ class MTPHead(torch.nn.Module):
         eh = torch.empty(*embed.shape[:-1], 2 * H, dtype=embed.dtype, device=embed.device)
         self.pre_fc_norm_embedding(embed, out=eh[..., :H])
         self.pre_fc_norm_hidden(hidden, out=eh[..., H:])
-        x = torch.nn.functional.linear(eh, self.fc)
+        x = linear(eh, self.fc)
         res = None  # the pending residual: each layer's output is x + res
         for layer, c in zip(self.layers, cache):
             x, res = layer.forward_parts(x, res, c)

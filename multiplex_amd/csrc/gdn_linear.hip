@@ -28,8 +28,8 @@
 // the norm fused it beats the separate norm plus the library GEMM up to 16
 // rows (7.4-8.1 us against 12.6-13.4 us) and loses beyond (at 64 rows every
 // workgroup re-reads y and z for its K slice, twice the weight bytes it
-// streams); the plain projection never beats the library.  Callers dispatch
-// on that.
+// streams).  The plain projection beats the library only up to 16 rows, in
+// linear_rows16_kernel.  Callers dispatch on that.
 //
 // The slices of one tile meet without fences.  Each workgroup writes its
 // partial tile with device-coherent stores (cache policy sc1, the encoding
@@ -289,6 +289,127 @@ linear_decode_kernel(const LinParams p) {
   }
 }
 
+// ------------------------------------------------------------ up to 16 rows
+//
+// The plain projection of at most 16 rows: a workgroup forms a whole tile of
+// 16 NB columns.  Its four waves take 128-wide chunks of K in turn (two chunks'
+// operands in flight each) and their partial tiles are summed once in LDS, so
+// no slices meet in memory: no workspace, no ticket.
+// Reading the weights bounds it.  A is read from the L2 by every workgroup, as
+// many bytes as its weights at NB = 1 and 16 rows, so a workgroup is as wide as
+// keeps the CUs evenly busy (rows16_blocks), and the workgroups of an XCD start
+// at different chunks, so that they do not all read the same lines of A at once
+// (24576 x 4096 at 16 rows, 64 columns: 43 us without, 36 with).
+// Graph-replayed at 4 rows against the sliced kernel below 64 columns and the
+// library (us; 16 rows in brackets):
+//   12352 x 2048 (NB = 4)  11.3 (11.9), 14.1 (14.4), 11.5 (11.5)
+//   10240 x 4096 (NB = 3)  15.6 (17.2), 17.7 (20.2), 18.7 (20.2)
+//    4096 x 4096 (NB = 1)   8.0  (9.8),  9.9 (10.5), 11.9 (12.3)
+//   24576 x 4096 (NB = 3)  34.1 (31.9), 35.5 (37.7), 34.4 (34.6)
+//    2048 x 4096 (NB = 1)   8.4  (9.7),  7.5  (7.8),  8.5  (8.6): half the CUs idle, so N <= 2048 is sliced
+// (84 MB in 15.6 us: 5.4 TB/s, the weights in the last-level cache).
+template <int NB>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1))) void linear_rows16_kernel(const LinParams p) {
+  constexpr int KC = 128, SQ = KC / 32;  // columns of K per chunk, k-steps
+  constexpr int PF = 2;                  // chunks in flight per wave
+  const int n0 = blockIdx.x * 16 * NB;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lr = lane & 15, lq = lane >> 4, lg8 = lq * 8;
+  const int nch = p.K / KC;  // a multiple of 4 (K is one of 512): n chunks for each wave
+  const int n = nch / 4;
+  const int rot = static_cast<int>(blockIdx.x / kXcds) % nch;
+
+  __shared__ __align__(16) float red[4][NB][64][4];  // each wave's partial tile, lane-major
+
+  const uint16_t* wp[NB];
+#pragma unroll
+  for (int b = 0; b < NB; ++b) wp[b] = p.w + static_cast<int64_t>(min(n0 + 16 * b + lr, p.N - 1)) * p.K + lg8;
+  // rows past M re-read row M - 1; their sums are never stored
+  const uint16_t* xp = p.x + static_cast<int64_t>(min(lr, p.M - 1)) * p.ldx + lg8;
+
+  bf16x8 wf[PF][NB][SQ], af[PF][SQ];
+  auto load = [&](int j, int i) {
+    int c = 4 * i + wave + rot;
+    c = (c >= nch ? c - nch : c) * KC;
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+      for (int s = 0; s < SQ; ++s) wf[j][b][s] = ld_bf16x8(wp[b] + c + 32 * s);
+#pragma unroll
+    for (int s = 0; s < SQ; ++s) af[j][s] = ld_bf16x8(xp + c + 32 * s);
+  };
+  f32x4 acc[NB];
+#pragma unroll
+  for (int b = 0; b < NB; ++b) acc[b] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  auto compute = [&](int j) {
+#pragma unroll
+    for (int s = 0; s < SQ; ++s)
+#pragma unroll
+      for (int b = 0; b < NB; ++b) acc[b] = mfma16(wf[j][b][s], af[j][s], acc[b]);
+  };
+#pragma unroll
+  for (int j = 0; j < PF; ++j) load(j, min(j, n - 1));
+  __builtin_amdgcn_sched_barrier(0);  // every load above is issued before the first wait
+  int i0 = 0;
+  for (; i0 + PF < n; i0 += PF) {
+#pragma unroll
+    for (int j = 0; j < PF; ++j) {
+      compute(j);
+      load(j, min(i0 + PF + j, n - 1));
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < PF; ++j)
+    if (i0 + j < n) compute(j);
+
+#pragma unroll
+  for (int b = 0; b < NB; ++b) *reinterpret_cast<f32x4*>(red[wave][b][lane]) = acc[b];
+  __syncthreads();
+  // wave b sums block b: lane (lr, lq) holds out[lr][n0 + 16 b + 4 lq + i]
+  static_assert(NB <= 4, "one wave per column block");
+  if (wave >= NB) return;
+  f32x4 sum = *reinterpret_cast<const f32x4*>(red[0][wave][lane]);
+#pragma unroll
+  for (int w = 1; w < 4; ++w) sum += *reinterpret_cast<const f32x4*>(red[w][wave][lane]);
+  const int c = n0 + 16 * wave + 4 * lq;
+  if (lr < p.M && c < p.N)
+    *reinterpret_cast<u32x2*>(p.out + lr * p.ldo + c) = u32x2{pk_bf16(sum[0], sum[1]), pk_bf16(sum[2], sum[3])};
+}
+
+// Up to one 16-column tile per two CUs the sliced kernel's K split fills the
+// chip and is the faster one (its comment has both at 2048 columns).
+constexpr int kCUs = 256;
+constexpr int64_t kSlicedN = 8 * kCUs;
+
+// 16-column blocks per workgroup: as many, up to 4, as give the busiest CU
+// the fewest blocks, and of those the most.
+int rows16_blocks(int64_t N) {
+  int best = 1;
+  int64_t fewest = INT64_MAX;
+  for (int nb = 1; nb <= 4; ++nb) {
+    const int64_t tiles = (N + 16 * nb - 1) / (16 * nb);
+    const int64_t blocks = (tiles + kCUs - 1) / kCUs * nb;
+    if (blocks <= fewest) {
+      best = nb;
+      fewest = blocks;
+    }
+  }
+  return best;
+}
+
+void launch_rows16(const LinParams& p, hipStream_t st) {
+  const int nb = rows16_blocks(p.N);
+  const dim3 grid(static_cast<unsigned>((p.N + 16 * nb - 1) / (16 * nb)));
+  switch (nb) {
+    case 1: hipLaunchKernelGGL(linear_rows16_kernel<1>, grid, dim3(256), 0, st, p); break;
+    case 2: hipLaunchKernelGGL(linear_rows16_kernel<2>, grid, dim3(256), 0, st, p); break;
+    case 3: hipLaunchKernelGGL(linear_rows16_kernel<3>, grid, dim3(256), 0, st, p); break;
+    default: hipLaunchKernelGGL(linear_rows16_kernel<4>, grid, dim3(256), 0, st, p); break;
+  }
+}
+
 // Row blocks per workgroup: 16-row blocks, as few as cover M, so small
 // batches hold fewer registers and less LDS and more workgroups share a CU.
 int row_blocks(int64_t M) { return M <= 16 ? 1 : M <= 32 ? 2 : 4; }
@@ -374,6 +495,10 @@ extern "C" int gdn_linear_decode(const void* x, int64_t ldx, const void* gate, i
   p.KSL = static_cast<int>(ksl);
   const dim3 grid(static_cast<unsigned>((nt + kXcds - 1) / kXcds * kXcds * ksl));
   hipStream_t st = static_cast<hipStream_t>(stream);
+  if (!norm && M <= 16 && N > kSlicedN) {
+    launch_rows16(p, st);
+    return gdn_host::check_launch("gdn_linear_decode");
+  }
   const bool wf32 = norm_w_dtype == GDN_DTYPE_F32;
   switch (row_blocks(M)) {
     case 1: launch<1>(p, norm, head_dim, wf32, grid, st); break;
@@ -381,4 +506,31 @@ extern "C" int gdn_linear_decode(const void* x, int64_t ldx, const void* gate, i
     default: launch<4>(p, norm, head_dim, wf32, grid, st); break;
   }
   return gdn_host::check_launch("gdn_linear_decode");
+}
+
+extern "C" int gdn_linear_rows16(const void* x, int64_t ldx, const void* W, void* out, int64_t ldo, int64_t M,
+                                 int64_t N, int64_t K, void* stream) {
+  using gdn_host::fail;
+  if (M < 1 || M > 16) return fail(GDN_ERR_UNSUPPORTED, "gdn_linear_rows16: M=%lld outside [1, 16]", (long long)M);
+  if (K < LK || K % LK != 0 || K > INT32_MAX)
+    return fail(GDN_ERR_UNSUPPORTED, "gdn_linear_rows16: K=%lld is not a multiple of %d", (long long)K, LK);
+  if (N < 1 || N % 8 != 0 || N > kMaxN)
+    return fail(GDN_ERR_UNSUPPORTED, "gdn_linear_rows16: N=%lld must be a positive multiple of 8 up to %lld",
+                (long long)N, (long long)kMaxN);
+  if (!x || !W || !out) return fail(GDN_ERR_INVALID, "gdn_linear_rows16: null pointer");
+  if (ldx < K || ldo < N || ldx % 8 != 0 || ldo % 8 != 0)
+    return fail(GDN_ERR_INVALID, "gdn_linear_rows16: row strides must cover the rows and be multiples of 8");
+  if (!gdn_host::aligned(x, 16) || !gdn_host::aligned(W, 16) || !gdn_host::aligned(out, 16))
+    return fail(GDN_ERR_INVALID, "gdn_linear_rows16: pointers must be 16-byte aligned");
+  LinParams p = {};
+  p.x = static_cast<const uint16_t*>(x);
+  p.ldx = ldx;
+  p.w = static_cast<const uint16_t*>(W);
+  p.out = static_cast<uint16_t*>(out);
+  p.ldo = ldo;
+  p.M = static_cast<int>(M);
+  p.N = static_cast<int>(N);
+  p.K = static_cast<int>(K);
+  launch_rows16(p, static_cast<hipStream_t>(stream));
+  return gdn_host::check_launch("gdn_linear_rows16");
 }

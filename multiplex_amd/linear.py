@@ -11,10 +11,12 @@ so the norm's output is never written.
 Graph-replayed against the separate norm kernel plus hipBLASLt at hidden
 2048, the fused norm + out_proj takes 7.4-8.1 us against 12.6-13.4 us up to
 16 rows, and loses beyond (11.4 against 10.9 us at 32 rows, 16.4 against
-13.1 us at 64); the plain projection is 1-2 us slower than the library at
-every row count.  So the mixer uses ``gated_norm_linear_decode`` up to
-``FUSED_NORM_MAX_ROWS`` rows and the library elsewhere; ``linear_decode``
-(the same kernel without the norm) is the unfused reference for tests.
+13.1 us at 64).  So the mixer uses ``gated_norm_linear_decode`` up to
+``FUSED_NORM_MAX_ROWS`` rows; ``linear_decode`` (the same kernel without the
+norm) is the unfused reference for tests.
+
+:func:`linear` is the layers' plain projection: up to 16 rows
+``gdn_linear_rows16``, the library beyond.
 
 The kernel sums its K slices through a workspace of fp32 partials and one
 ticket per output tile; the tickets must start at zero and every call
@@ -32,7 +34,7 @@ import torch
 from . import _lib
 from .gated_delta import _dtype_code, _ptr, _require_device, _stream
 
-__all__ = ["DECODE_MAX_ROWS", "FUSED_NORM_MAX_ROWS", "DecodeWorkspace", "linear_decode",
+__all__ = ["linear", "DECODE_MAX_ROWS", "FUSED_NORM_MAX_ROWS", "DecodeWorkspace", "linear_decode",
            "gated_norm_linear_decode", "linear_decode_workspace_bytes", "decode_shape_ok"]
 
 DECODE_MAX_ROWS = 64
@@ -98,6 +100,34 @@ def _launch(x, gate, norm_weight, eps, head_dim, weight, out, workspace):
     _lib.call("gdn_linear_decode", _ptr(x), ldx, _ptr(gate), ldg, _ptr(norm_weight), nw_dt, float(eps),
               int(head_dim), _ptr(weight), _ptr(out), ldo, M, N, K, _ptr(ws), ws.numel(), _stream(dev))
     return out
+
+
+def linear(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
+    """``x @ weight.T`` (``torch.nn.functional.linear`` without a bias).
+
+    Up to 16 rows of bf16, K a multiple of 512 up to 4096 and N a multiple of
+    8 above 2048, by ``gdn_linear_rows16``; the library elsewhere, and where
+    autograd, autocast or a tensor subclass needs its operator.  The line:
+    graph-replayed at 4 (16) rows, 4096 x 4096 takes 8.0 (9.8) against 11.9
+    (12.3) us, 10240 x 4096 15.6 (17.2) against 18.7 (20.2), 12352 x 2048
+    11.3 (11.9) against 11.5 (11.5); with K = 8192 or 12288 at 4096 columns
+    the library is 1 us faster, and at 2048 columns as fast.  The library
+    call itself costs the host 19 us, the launch 4.
+    """
+    N, K = weight.shape
+    rows = x.numel() // K if K else 0
+    if (1 <= rows <= 16 and 512 <= K <= 4096 and K % 512 == 0 and N > 2048 and N % 8 == 0
+            and x.dtype is torch.bfloat16 and weight.dtype is torch.bfloat16 and x.is_cuda and weight.is_cuda
+            and x.shape[-1] == K and x.is_contiguous() and weight.is_contiguous()
+            and type(x) is torch.Tensor and type(weight) in (torch.Tensor, torch.nn.Parameter)
+            and x.device == weight.device and not torch.is_autocast_enabled()
+            and not (torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad))):
+        xp, wp = x.data_ptr(), weight.data_ptr()
+        if xp % 16 == 0 and wp % 16 == 0:
+            out = torch.empty(*x.shape[:-1], N, dtype=torch.bfloat16, device=x.device)
+            _lib.call("gdn_linear_rows16", xp, K, wp, out.data_ptr(), N, rows, N, K, _stream(x.device))
+            return out
+    return torch.nn.functional.linear(x, weight)
 
 
 def linear_decode(x: torch.Tensor, weight: torch.Tensor, *, out: Optional[torch.Tensor] = None,

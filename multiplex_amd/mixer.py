@@ -11,8 +11,9 @@ kernels update in place.  With pooled states a decode step (one token per
 row) also updates the conv state ``cache[0]`` in place.
 
 Data path per call:
-  in_proj_qkv / z / b / a      one library GEMM (hipBLASLt through torch); the
-                               kernels below read its column slices in place
+  in_proj_qkv / z / b / a      one GEMM (``gdn_linear_rows16`` up to 16 rows, else
+                               hipBLASLt through torch); the kernels below read
+                               its column slices in place
   gdn_conv_prologue            fused conv1d + SiLU + q/k norm (HIP)
   gated_delta_update           recurrent or chunked kernel (HIP); where the
                                chunked kernel runs (long unmasked rows) the
@@ -45,7 +46,7 @@ from .conv import conv_state_commit, gdn_conv_chunked, gdn_conv_prologue
 from .epilogue import gated_rms_norm
 from .state_pool import PooledBatch
 from .gated_delta import CHUNK_MIN_TOKENS, IntSeq, gated_delta_commit, gated_delta_update, gated_delta_verify
-from .linear import FUSED_NORM_MAX_ROWS, DecodeWorkspace, decode_shape_ok, gated_norm_linear_decode
+from .linear import FUSED_NORM_MAX_ROWS, DecodeWorkspace, decode_shape_ok, gated_norm_linear_decode, linear
 
 __all__ = ["GatedDeltaNet", "gated_rms_norm", "commit_verified"]
 
@@ -153,7 +154,7 @@ class GatedDeltaNet(torch.nn.Module):
         w = self._fused_in_proj_weight()
         c1, c2, c3 = self._splits
         if B * S <= 256:
-            out = torch.nn.functional.linear(inputs, w)
+            out = linear(inputs, w)
             qkv, z, ba = out[..., :c1], out[..., c1:c2], out[..., c2:]
         else:
             out = torch.nn.functional.linear(inputs, w[:c2])

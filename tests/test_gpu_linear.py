@@ -48,6 +48,36 @@ def test_linear_decode_matches_float64(M, N, K):
     assert rel_err(_np(out), ref) <= 1e-3
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 2056, 512), (16, 4096, 4096), (5, 4104, 1536), (16, 8200, 512),
+                                   (7, 10240, 4096), (3, 12352, 2048), (16, 24584, 1024)])
+def test_linear_up_to_16_rows_matches_float64(M, N, K):
+    """One workgroup per tile of 16 to 64 columns: tiles with a ragged last one,
+    one to eight chunks of K a wave.  fp32 sums in another order, as above."""
+    gen = torch.Generator().manual_seed(M + N + K)
+    x, W = _bf16(gen, M, K), _bf16(gen, N, K, scale=K ** -0.5)
+    xd, Wd = x.to(DEV), W.to(DEV)
+    out = lin.linear(xd.view(M, 1, K), Wd)
+    guard = torch.zeros(M + 1, N + 8, dtype=torch.bfloat16, device=DEV)
+    mx.linear_decode(xd, Wd, out=guard[:M, :N])
+    torch.cuda.synchronize()
+    ref = gdn.bf16_round(_np(x) @ _np(W).T)
+    assert rel_err(_np(out).reshape(M, N), ref) <= 1e-3
+    assert torch.equal(out.view(M, N), guard[:M, :N])
+    assert not guard[M:].any() and not guard[:, N:].any()
+
+
+def test_linear_leaves_other_calls_to_the_library():
+    """Rows, types and layouts the kernel does not take, and calls that record a gradient."""
+    gen = torch.Generator().manual_seed(95)
+    W = _bf16(gen, 4096, 1024, scale=1 / 32).to(DEV)
+    for x in (_bf16(gen, 17, 1024).to(DEV), _bf16(gen, 4, 2048).to(DEV)[:, ::2], _bf16(gen, 0, 1024).to(DEV),
+              _bf16(gen, 4 * 1024 + 1).to(DEV)[1:].view(4, 1024)):
+        assert torch.equal(lin.linear(x, W), torch.nn.functional.linear(x, W))
+    x = _bf16(gen, 4, 1024).to(DEV).requires_grad_()
+    lin.linear(x, W).sum().backward()
+    assert x.grad is not None
+
+
 def test_linear_decode_reads_column_slices_and_writes_strided_rows():
     """x a column slice of a wider buffer, out rows inside a wider buffer."""
     gen = torch.Generator().manual_seed(91)
