@@ -379,6 +379,9 @@ int gdn_attn_fwd(const void* q, const void* qg, int64_t qg_ld, const void* k_cac
 int gdn_rms_norm(const void* x, const void* res, void* h_out, const void* w, int w_dtype, void* y,
                  int64_t y_ld, int64_t rows, int64_t D, float eps, void* stream);
 
+/* A KV cache's offsets: pos[b] = max(pos[b] + delta, lo) for B rows. */
+int gdn_pos_add(int32_t* pos, int64_t B, int32_t delta, int32_t lo, void* stream);
+
 /* The MLP activation: out[r, i] = silu(gate_up[r, i]) * gate_up[r, I + i]
  * (bf16; gate_up is one [rows, 2I] product of the gate and up projections). */
 int gdn_silu_mul(const void* gate_up, void* out, int64_t rows, int64_t I, void* stream);

@@ -48,6 +48,7 @@ EXPORTS = (
     "gdn_attn_workspace_bytes",
     "gdn_attn_fwd",
     "gdn_rms_norm",
+    "gdn_pos_add",
     "gdn_silu_mul",
     "gdn_linear_decode_workspace_bytes",
     "gdn_linear_rows16",
@@ -170,6 +171,7 @@ _SIGNATURES = {
         [_P, _P, _I64, _P, _P, _P, _P, c_float, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _P, c_size_t, _P],
     ),
     "gdn_rms_norm": (c_int, [_P, _P, _P, _P, c_int, _P, _I64, _I64, _I64, c_float, _P]),
+    "gdn_pos_add": (c_int, [_P, _I64, c_int32, c_int32, _P]),
     "gdn_silu_mul": (c_int, [_P, _P, _I64, _I64, _P]),
     "gdn_linear_decode_workspace_bytes": (c_size_t, [_I64, _I64, _I64]),
     "gdn_linear_rows16": (c_int, [_P, _I64, _P, _P, _I64, _I64, _I64, _I64, _P]),

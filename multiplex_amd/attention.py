@@ -324,15 +324,27 @@ class KVCache:
             setattr(self, name, new)
 
     def advance(self, T: int) -> None:
-        self.lengths = [n + int(T) for n in self.lengths]
-        self.pos0.add_(int(T))
+        T = int(T)
+        self.lengths = [n + T for n in self.lengths]
+        if not self._pos_add(T, -2**31):
+            self.pos0.add_(T)
 
     def trim(self, n: int) -> int:
         """Drops the last ``n`` positions of every row (the drafter's rollback)."""
         n = min(int(n), self.offset)
         self.lengths = [max(0, m - n) for m in self.lengths]
-        self.pos0.sub_(n).clamp_(min=0)
+        if not self._pos_add(-n, 0):
+            self.pos0.sub_(n).clamp_(min=0)
         return n
+
+    def _pos_add(self, delta: int, lo: int) -> bool:
+        """``pos0 = max(pos0 + delta, lo)`` in one launch (``gdn_pos_add``), or
+        False for offsets the kernel does not take (e.g. on the host)."""
+        p = self.pos0
+        if not p.is_cuda or p.dtype is not torch.int32 or not p.is_contiguous() or not -2**31 <= delta < 2**31:
+            return False
+        _lib.call("gdn_pos_add", p.data_ptr(), p.numel(), delta, lo, _stream(p.device))
+        return True
 
     def filter(self, keep: Sequence[int]) -> None:
         """Keeps rows ``keep`` (a batch leave)."""

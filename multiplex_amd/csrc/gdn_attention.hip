@@ -28,6 +28,7 @@
 //                        out when a gate is given.
 //   rms_norm_kernel      the layers' RMSNorm over the hidden size, optionally of
 //                        a residual sum it also writes out.
+//   pos_add_kernel       the cache offsets' advance and rollback.
 //   silu_mul_kernel      the MLP's silu(gate) * up.
 #include <cfloat>
 
@@ -1099,6 +1100,16 @@ __global__ __launch_bounds__(256) void rms_norm_kernel(const uint16_t* x, const 
   }
 }
 
+// ------------------------------------------------------------ pos_add
+
+// pos[b] = max(pos[b] + delta, lo): a KV cache's advance and rollback, one
+// launch each (the rollback was a subtraction and a clamp, two launches of
+// 1.5 us and 4 us of host time for a few integers).
+__global__ __launch_bounds__(256) void pos_add_kernel(int32_t* pos, int B, int32_t delta, int32_t lo) {
+  const int b = blockIdx.x * 256 + threadIdx.x;
+  if (b < B) pos[b] = max(static_cast<int32_t>(static_cast<uint32_t>(pos[b]) + static_cast<uint32_t>(delta)), lo);
+}
+
 // ------------------------------------------------------------ silu_mul
 
 // out[r, i] = silu(gu[r, i]) * gu[r, I + i]; 8 elements per thread.
@@ -1277,6 +1288,16 @@ extern "C" int gdn_rms_norm(const void* x, const void* res, void* h_out, const v
                      static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(res), static_cast<uint16_t*>(h_out),
                      w, w_dtype, static_cast<uint16_t*>(y), y_ld, static_cast<int>(D), eps);
   return gdn_host::check_launch("gdn_rms_norm");
+}
+
+extern "C" int gdn_pos_add(int32_t* pos, int64_t B, int32_t delta, int32_t lo, void* stream) {
+  using gdn_host::fail;
+  if (B < 0 || B > INT32_MAX) return fail(GDN_ERR_INVALID, "gdn_pos_add: bad sizes");
+  if (B == 0) return GDN_OK;
+  if (!pos) return fail(GDN_ERR_INVALID, "gdn_pos_add: null pointer");
+  hipLaunchKernelGGL(pos_add_kernel, dim3(static_cast<unsigned>((B + 255) / 256)), dim3(256), 0,
+                     static_cast<hipStream_t>(stream), pos, static_cast<int>(B), delta, lo);
+  return gdn_host::check_launch("gdn_pos_add");
 }
 
 extern "C" int gdn_silu_mul(const void* gate_up, void* out, int64_t rows, int64_t I, void* stream) {

@@ -208,6 +208,26 @@ def test_attention_matches_oracle(name):
     assert _row_errs(got, ref).max() < ATT_TOL
 
 
+@pytest.mark.parametrize("B", [1, 256, 257])
+def test_cache_offsets_advance_and_roll_back(B):
+    """Exact: the device offsets follow the host lengths, and a rollback stops
+    each row at zero."""
+    c = mx.KVCache(B, 1, 128, 256, DEV)
+    c.lengths = [b % 7 for b in range(B)]
+    c.pos0.copy_(torch.tensor(c.lengths, dtype=torch.int32))
+    for step in (3, -5, 9, -20):
+        if step > 0:
+            c.advance(step)
+        else:
+            c.trim(-step)
+        assert c.pos0.tolist() == c.lengths
+    big = torch.tensor([2**31 - 1, -2**31 + 3], dtype=torch.int32, device=DEV)  # wraps as torch's add_ does
+    c = mx.KVCache(2, 1, 128, 256, DEV)
+    c.pos0 = big.clone()
+    c.advance(5)
+    assert torch.equal(c.pos0, big.add(5))
+
+
 def test_split_keys_agree_with_one_range():
     """A 2000-key decode split over 1 and 5 workgroups per row."""
     gen = torch.Generator().manual_seed(73)
