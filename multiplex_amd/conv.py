@@ -16,7 +16,7 @@ import torch
 
 from . import _lib
 from .gated_delta import (CHUNK, IntSeq, PreparedCall, _contig, _cu_seqlens, _dtype_code, _gate_codes, _gate_pair,
-                          _int_rows, _mask_u8, _param_codes, _ptr, _require_device, _state_operands, _stream,
+                          _int_rows, _mask_u8, _on_device, _param_codes, _ptr, _require_device, _state_operands, _stream,
                           _token_rows)
 
 __all__ = ["gdn_conv_prologue", "prepare_conv_prologue", "conv_state_commit", "gdn_conv_chunked",
@@ -114,7 +114,7 @@ def gdn_conv_prologue(qkv: torch.Tensor, conv_weight: torch.Tensor, num_k_heads:
     """
     args, _keep, outs, dev = _prologue_args(qkv, conv_weight, num_k_heads, num_v_heads, head_k_dim, head_v_dim,
                                             conv_state, mask, cu_seqlens, eps, write_conv_state, conv_state_out)
-    with torch.cuda.device(dev):
+    with _on_device(dev):
         _lib.call("gdn_conv_prologue", *args)
     return outs
 
@@ -158,7 +158,7 @@ def conv_state_commit(conv_state: Optional[torch.Tensor], qkv: torch.Tensor, n_c
     ld = _token_rows(qkv, C)
     if ld is None:
         qkv, ld = qkv.contiguous(), C
-    with torch.cuda.device(dev):
+    with _on_device(dev):
         _lib.call("gdn_conv_state_commit", _ptr(conv_state), _ptr(qkv), io, ld, _ptr(m), _ptr(n), _ptr(out),
                   B, T, C, Kt, _stream(dev))
     return out
@@ -239,7 +239,7 @@ def gdn_conv_chunked(qkv: torch.Tensor, conv_weight: torch.Tensor, num_k_heads: 
     args, _keep, outs, dev = _conv_chunked_args(qkv, conv_weight, num_k_heads, num_v_heads, head_k_dim,
                                                 head_v_dim, a, b, A_log, dt_bias, state, conv_state, cu_seqlens,
                                                 eps, state_out, workspace, state_index, write_conv_state)
-    with torch.cuda.device(dev):
+    with _on_device(dev):
         _lib.call("gdn_chunk_fwd_conv", *args)
     return outs
 

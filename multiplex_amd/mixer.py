@@ -152,17 +152,15 @@ class GatedDeltaNet(torch.nn.Module):
         """
         B, S, _ = inputs.shape
         w = self._fused_in_proj_weight()
-        c1, c2, c3 = self._splits
+        c1, c2, _ = self._splits
+        hv = self.num_v_heads
         if B * S <= 256:
-            out = linear(inputs, w)
-            qkv, z, ba = out[..., :c1], out[..., c1:c2], out[..., c2:]
+            qkv, z, b, a = linear(inputs, w).split((c1, c2 - c1, hv, hv), -1)
         else:
             out = torch.nn.functional.linear(inputs, w[:c2])
             ba = torch.nn.functional.linear(inputs, w[c2:])
-            qkv, z = out[..., :c1], out[..., c1:]
-        z = z.unflatten(-1, (self.num_v_heads, self.head_v_dim))
-        hv = self.num_v_heads
-        return qkv, z, ba[..., hv:], ba[..., :hv]
+            (qkv, z), (b, a) = out.split((c1, c2 - c1), -1), ba.split((hv, hv), -1)
+        return qkv, z.view(B, S, hv, self.head_v_dim), a, b
 
     def _epilogue(self, y, z):
         B, S = y.shape[:2]
