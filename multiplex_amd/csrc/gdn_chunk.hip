@@ -445,10 +445,10 @@ __device__ __forceinline__ double wave_scan_d(double x) {
 }
 
 // KT_LDS: the scan forms K^T from K in LDS, so the record carries no K^T.
-// Four workgroups per CU: 35.6 KB of LDS each and at most 128 VGPRs (four
-// waves per SIMD; left to itself the compiler takes 137-138, which leaves
-// three).  At 4096 tokens x 32 heads the 2048 workgroups then run in two
-// full rounds instead of two and two thirds.
+// Four heads per CU: 35.6 KB of LDS each and at most 128 VGPRs (four waves per
+// SIMD; left to itself the compiler takes 137-138, which leaves three).  At
+// 4096 tokens x 32 heads the 2048 heads then run in two full rounds instead of
+// two and two thirds.
 //
 // CONV (1: bf16 taps, 2: fp32 taps): the conv prologue is fused in.  The
 // workgroup forms its chunk's q and k rows (its k-head) and v rows (its
@@ -457,52 +457,67 @@ __device__ __forceinline__ double wave_scan_d(double x) {
 // slot of an empty packed sequence passes its conv state through.
 //
 // MASK: a token mask is given (the unmasked kernels carry none of its code).
-template <bool KT_LDS, int CONV, bool MASK>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void chunk_prep_kernel(const ChunkParams p) {
-  // Two 17 KB buffers, each reused once (LDS stays under 40 KB, so four
-  // workgroups fit on a CU):  buf0 = K rows, then A;  buf1 = Q rows, then
-  // the P hi/lo planes in fragment order, then (I + A)^{-1}.  The extra last
-  // workgroup of a packed call orders the sequences in buf0 instead.
+//
+// NH = 2 (an even number of v-heads per k-head): a workgroup of eight waves
+// takes two v-heads of one k-head.  Their q and k rows are then loaded (or, with
+// CONV, convolved, SiLU'd and normalised: two thirds of the conv's vector work,
+// a large part of the fused prep's time) once for both instead of twice.  Where
+// it runs: the dispatch's comment.
+template <bool KT_LDS, int CONV, bool MASK, int NH>
+__global__ __launch_bounds__(256 * NH) __attribute__((amdgpu_waves_per_eu(4))) void chunk_prep_kernel(
+    const ChunkParams p) {
+  // Two 17 KB buffers per v-head, each reused once (LDS stays under 40 KB a
+  // head, so sixteen waves fit on a CU):  buf0 = K rows (head 0's), then A;
+  // buf1 = Q rows (head 0's), then the P hi/lo planes in fragment order, then
+  // (I + A)^{-1}.  The extra last workgroup of a packed call orders the
+  // sequences in buf0 instead.
+  constexpr int NT = 256 * NH;  // threads
   constexpr int kBuf = CH * KP * 2;
   static_assert(kBuf == CH * (CH + 4) * 4, "A and T must fill the K / Q buffers exactly");
   static_assert(kBuf >= 2 * CH * CH * 2, "P staging must fit in the Q buffer");
   static_assert(kBuf >= kOrderMax * 4, "the sequence lengths must fit in buf0");
-  __shared__ __align__(16) unsigned char buf0[kBuf];
-  __shared__ __align__(16) unsigned char buf1[kBuf];
+  __shared__ __align__(16) unsigned char bufs[NH][2][kBuf];
   if (p.order != nullptr && blockIdx.x == gridDim.x - 1) {
-    order_sequences(p, reinterpret_cast<int*>(buf0));
+    order_sequences(p, reinterpret_cast<int*>(bufs[0][0]));
     return;
   }
-  // work index = chunk * Hv + hv: both v-heads of a k-head (GQA) share an XCD
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform
+  const int hsel = NH == 2 ? wave >> 2 : 0;  // the wave's v-head of the workgroup's, and its place among
+  const int w4 = wave & 3, tid4 = tid & 255;  // that head's four waves (256 threads)
+  // work index = chunk * (Hv / NH) + hv0 / NH: the v-heads of a k-head (GQA) share an XCD
   const int w = xcd_work_index(gridDim.x - (p.order != nullptr ? 1 : 0));
-  const int c = w / p.Hv;
-  const int hv = w % p.Hv;
-  const int hk = hv / p.group;
-  const bool first_v = hv % p.group == 0;  // writes the k-head's K^T, K and Q
+  const int per_chunk = p.Hv / NH;
+  const int c = w / per_chunk;
+  const int hv0 = w % per_chunk * NH;
+  const int hv = hv0 + hsel;
+  const int hk = hv0 / p.group;
+  const bool first_v = hv0 % p.group == 0;  // writes the k-head's K^T, K and Q (into hv0's record)
   ChunkPos cp;
   if (!chunk_at(p, c, cp)) {
     if constexpr (CONV != 0) {
       if (p.cu != nullptr && cp.seq_len == 0 && cp.ci == 0)
-        conv_state_rows(p, cp.seq, cp.seq_tok0, 0, hk, hv, first_v, threadIdx.x);
+        conv_state_rows(p, cp.seq, cp.seq_tok0, 0, hk, hv, first_v && hsel == 0, tid4);
     }
     return;
   }
   const int64_t tok0 = cp.tok0;
   const int len = cp.len;
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform
   const int lr = lane & 15, lq = lane >> 4, lg8 = lq * 8;
 
-  __shared__ __align__(16) double Ld[CH];  // L_t log2(e) (the decays' exponents, base 2)
-  __shared__ float Bs[CH];
-  __shared__ float Ys[MASK ? CH : 1];  // 1, or 0 at a masked token (its row of P is zero)
-  auto Ks = reinterpret_cast<uint16_t(*)[KP]>(buf0);
-  auto Qs = reinterpret_cast<uint16_t(*)[KP]>(buf1);
-  auto As = reinterpret_cast<float(*)[CH + 4]>(buf0);
-  auto Ti = reinterpret_cast<float(*)[CH + 4]>(buf1);
-  uint16_t* Pst = reinterpret_cast<uint16_t*>(buf1);
+  __shared__ __align__(16) double Lds[NH][CH];  // L_t log2(e) (the decays' exponents, base 2)
+  __shared__ float Bss[NH][CH];
+  __shared__ float Yss[NH][MASK ? CH : 1];  // 1, or 0 at a masked token (its row of P is zero)
+  double* Ld = Lds[hsel];
+  float* Bs = Bss[hsel];
+  float* Ys = Yss[hsel];
+  auto Ks = reinterpret_cast<uint16_t(*)[KP]>(bufs[0][0]);
+  auto Qs = reinterpret_cast<uint16_t(*)[KP]>(bufs[0][1]);
+  auto As = reinterpret_cast<float(*)[CH + 4]>(bufs[hsel][0]);
+  auto Ti = reinterpret_cast<float(*)[CH + 4]>(bufs[hsel][1]);
+  uint16_t* Pst = reinterpret_cast<uint16_t*>(bufs[hsel][1]);
 
-  // Gate loads first, raw (wave 0 uses them; every wave issues them, so no
+  // Gate loads first, raw (a head's wave 0 uses them; every wave issues them, so no
   // branch lets the compiler start converting them early, which would wait),
   // so waiting for them does not wait for the K/Q rows queued behind; then
   // the rows (rows past the chunk's end read its last row and are zeroed at
@@ -513,12 +528,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void c
   float b_lane = 0.0f;
   bool on_lane = false;  // wave 0: token `lane` is real and not masked
   asm volatile("" ::: "memory");  // keeps the gate loads issued ahead of the rows
-  u32x4 kr[4], qr[4];
-  bool kq_on[4];  // the row is a real token (and, with MASK, not masked)
+  constexpr int RPT = 4 / NH;  // K (and Q) pieces per thread
+  u32x4 kr[RPT], qr[RPT];
+  bool kq_on[RPT];  // the row is a real token (and, with MASK, not masked)
   if constexpr (CONV == 0) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int i = tid + 256 * j;
+    for (int j = 0; j < RPT; ++j) {
+      const int i = tid + NT * j;
       const int r = i / (DK / 8), cc = (i % (DK / 8)) * 8;
       const int64_t off = ((tok0 + min(r, len - 1)) * p.Hk + hk) * DK + cc;
       kr[j] = *reinterpret_cast<const u32x4*>(p.k + off);
@@ -531,7 +547,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void c
     }
   }
   unsigned char* rec = p.ws + (static_cast<size_t>(c) * p.Hv + hv) * kRecBytes;
-  if (wave == 0) {
+  unsigned char* rec_k = p.ws + (static_cast<size_t>(c) * p.Hv + hv0) * kRecBytes;
+  if (w4 == 0) {
     float lg, bt;
     log_gates(p.ga, gr, lg, bt);
     // padding and masked tokens: no decay, no write (a masked token keeps
@@ -547,41 +564,43 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void c
   }
   if constexpr (CONV == 0) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int i = tid + 256 * j;
+    for (int j = 0; j < RPT; ++j) {
+      const int i = tid + NT * j;
       const int r = i / (DK / 8), cc = (i % (DK / 8)) * 8;
       const u32x4 kv = row_or_zero(kq_on[j], kr[j]), qv = row_or_zero(kq_on[j], qr[j]);
       *reinterpret_cast<u32x4*>(&Ks[r][cc]) = kv;
       *reinterpret_cast<u32x4*>(&Qs[r][cc]) = qv;
       if (first_v) {
-        *reinterpret_cast<u32x4*>(reinterpret_cast<uint16_t*>(rec + kOffKf) + frag_elem(r, cc, DK / 32)) = kv;
-        *reinterpret_cast<u32x4*>(reinterpret_cast<uint16_t*>(rec + kOffQf) + frag_elem(r, cc, DK / 32)) = qv;
+        *reinterpret_cast<u32x4*>(reinterpret_cast<uint16_t*>(rec_k + kOffKf) + frag_elem(r, cc, DK / 32)) = kv;
+        *reinterpret_cast<u32x4*>(reinterpret_cast<uint16_t*>(rec_k + kOffQf) + frag_elem(r, cc, DK / 32)) = qv;
       }
     }
   } else {
-    // 16-lane row rw of the workgroup takes 4 tokens, [4 rw, 4 rw + 4), of
-    // one head, lane g of the row channels 8 g .. 8 g + 7 of it: q, then k
-    // (to LDS and the records, as the loads above would), then v (for the
-    // scan).
+    // q and k: 16-lane row rw of the workgroup takes RPT tokens, [RPT rw,
+    // RPT rw + RPT), of one head, lane g of the row channels 8 g .. 8 g + 7 of
+    // it (to LDS and the records, as the loads above would); then v of each
+    // head by its four waves, four tokens a row (for the scan).
     constexpr int WDT = CONV == 2 ? GDN_DTYPE_F32 : GDN_DTYPE_BF16;
-    const int rw = 4 * wave + lq, g = lr, t0 = 4 * rw;
+    const int g = lr;
 #pragma unroll
     for (int role = 0; role < 2; ++role) {
-      u32x4 o[4];
+      u32x4 o[RPT];
+      const int t0 = RPT * (4 * wave + lq);
       const float post = role == 0 ? 1.0f / static_cast<float>(DK) : rsqrtf(static_cast<float>(DK));
-      conv_run<WDT, 4, true>(p, cp, (role * p.Hk + hk) * DK + 8 * g, t0, post, o);
+      conv_run<WDT, RPT, true>(p, cp, (role * p.Hk + hk) * DK + 8 * g, t0, post, o);
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
+      for (int u = 0; u < RPT; ++u) {
         const int r = t0 + u;
         const u32x4 val = row_or_zero(r < len, o[u]);
         *reinterpret_cast<u32x4*>(role == 0 ? &Qs[r][8 * g] : &Ks[r][8 * g]) = val;
         if (first_v)
-          *reinterpret_cast<u32x4*>(reinterpret_cast<uint16_t*>(rec + (role == 0 ? kOffQf : kOffKf)) +
+          *reinterpret_cast<u32x4*>(reinterpret_cast<uint16_t*>(rec_k + (role == 0 ? kOffQf : kOffKf)) +
                                     frag_elem(r, 8 * g, DK / 32)) = val;
       }
     }
     {
       u32x4 o[4];
+      const int t0 = 4 * (4 * w4 + lq);
       conv_run<WDT, 4, false>(p, cp, 2 * p.Hk * DK + hv * DV + 8 * g, t0, 1.0f, o);
 #pragma unroll
       for (int u = 0; u < 4; ++u)
@@ -589,11 +608,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void c
           *reinterpret_cast<u32x4*>(p.v_out + ((tok0 + t0 + u) * p.Hv + hv) * DV + 8 * g) = o[u];
     }
     if (cp.ci == n_chunks(cp.seq_len) - 1)
-      conv_state_rows(p, cp.seq, cp.seq_tok0, cp.seq_len, hk, hv, first_v, tid);
+      conv_state_rows(p, cp.seq, cp.seq_tok0, cp.seq_len, hk, hv, first_v && hsel == 0, tid4);
   }
   __syncthreads();
 
-  // K K^T and Q K^T: wave w computes row block w (16 rows) x 4 column
+  // K K^T and Q K^T, by each head's four waves for itself (the matrix cores are
+  // idle otherwise): wave w computes row block w (16 rows) x 4 column
   // blocks, as the transposed products K_j K_w^T and K_j Q_w^T (an A and a
   // B fragment have the same layout, so the operands swap roles): lane
   // (r, q) of tile j then holds row 16w + r, columns 16j + 4q .. +3 (K K^T is
@@ -616,19 +636,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void c
   for (int h = 0; h < 2; ++h)
 #pragma unroll
     for (int e = 0; e < 8; ++e) eye[h][e] = static_cast<__bf16>(lg8 + e == lr + 16 * h ? 1.0f : 0.0f);
-  unsigned char* KTg = rec + kOffKT + (wave >> 1) * 1024 + (lr + 16 * (2 * (wave & 1) + (lq >> 1))) * 16 + (lq & 1) * 8;
+  unsigned char* KTg = rec_k + kOffKT + (w4 >> 1) * 1024 + (lr + 16 * (2 * (w4 & 1) + (lq >> 1))) * 16 + (lq & 1) * 8;
 #pragma unroll
   for (int s = 0; s < DK / 32; ++s) {
     const int kc = s * 32 + lg8;
-    const bf16x8 ak = lds8(&Ks[16 * wave + lr][kc]);
-    const bf16x8 aq = lds8(&Qs[16 * wave + lr][kc]);
+    const bf16x8 ak = lds8(&Ks[16 * w4 + lr][kc]);
+    const bf16x8 aq = lds8(&Qs[16 * w4 + lr][kc]);
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const bf16x8 bk = lds8(&Ks[16 * j + lr][kc]);
       kk[j] = mfma16(bk, ak, kk[j]);
       qk[j] = mfma16(bk, aq, qk[j]);
     }
-    if (!KT_LDS && first_v) {
+    if (!KT_LDS && first_v && hsel == 0) {
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
         const f32x4 t = mfma16(ak, eye[h], f32x4{0.0f, 0.0f, 0.0f, 0.0f});
@@ -644,7 +664,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void c
   // Decays, A (to LDS, fp32) and P (hi/lo bf16, staged in fragment order):
   // lane (r, q) takes row t = 16w + r, columns 16j + 4q .. +3.
   {
-    const int t = 16 * wave + lr;
+    const int t = 16 * w4 + lr;
     typedef double f64x2 __attribute__((ext_vector_type(2)));
     const double Lt = Ld[t];
     const float bt = Bs[t];
@@ -680,7 +700,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void c
   // the scan never reads them.
   const int dbase = 16 * (lane >> 4), dcol = lane & 15;
   float x[16];
-  if (wave == 0) {
+  if (w4 == 0) {
     float a[16][16];
 #pragma unroll
     for (int t = 1; t < 16; ++t)
@@ -694,14 +714,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void c
       x[t] = t < dcol ? 0.0f : acc;
     }
   } else {
-    for (int i = tid - 64; i < 1024; i += 192) {
+    for (int i = tid4 - 64; i < 1024; i += 192) {
       const int frag = (i & 511) >> 6;
       if (frag != 1 && frag != 3)
         *reinterpret_cast<u32x4*>(rec + kOffPh + 16 * i) = *reinterpret_cast<const u32x4*>(Pst + 8 * i);
     }
   }
   __syncthreads();  // the P planes are out: their buffer takes (I + A)^{-1}
-  if (wave == 0) {
+  if (w4 == 0) {
 #pragma unroll
     for (int t = 0; t < 16; ++t) Ti[dbase + t][dbase + dcol] = x[t];
   }
@@ -719,7 +739,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void c
   // no wave reads another's off-diagonal blocks until the barrier below.
   {
     const int ln = lane & 15, lk = lane >> 4;
-    const int J = wave;
+    const int J = w4;
     f32x4 tcol[3];  // T_{J+1,J} .. T_{J+3,J}
     float tjj[4];
 #pragma unroll
@@ -762,7 +782,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void c
   // fragments (rows < 32, columns >= 32) are not stored, as for P
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
-    const int i = tid + 256 * j;
+    const int i = tid4 + 256 * j;
     const int r = i >> 3, cc = (i & 7) * 8;
     if (r < 32 && cc >= 32) continue;
     const bool upper = (cc >> 4) > (r >> 4);
@@ -773,7 +793,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void c
     split4_store(b, Th + frag_elem(r, cc + 4, CH / 32), Tl + frag_elem(r, cc + 4, CH / 32));
   }
   // the gates' record entries (only the scan reads them)
-  if (wave == 0) {
+  if (w4 == 0) {
     const uint64_t u = __builtin_bit_cast(uint64_t, L_lane);
     const uint32_t lo = __builtin_amdgcn_readlane(static_cast<int>(u), 63);
     const uint32_t hi = __builtin_amdgcn_readlane(static_cast<int>(u >> 32), 63);
@@ -1408,22 +1428,34 @@ int chunk_fwd(const void* q, const void* k, const void* v, int qkv_dtype, int ga
   // operand bytes per CU); else the record's K^T (a shorter chain per chunk).
   const bool kt_lds = static_cast<int64_t>(kTiles) * n_seqs * Hv > kCUs;
   if ((phases & kPhasePrep) && chunks > 0) {
-    // one workgroup per (chunk slot, v-head), and one more that orders packed sequences
-    const dim3 grid(static_cast<unsigned>(chunks * Hv + (p.order != nullptr ? 1 : 0)));
+    // one workgroup per (chunk slot, v-head or pair of a k-head's), and one more that orders packed sequences
     // (the fused prologue takes no mask: conv != null implies mask == null)
     const int cv = conv == nullptr ? 0 : (conv->w_dtype == GDN_DTYPE_F32 ? 2 : 1);
-    const bool masked = mask != nullptr;
-    if (kt_lds) {
-      if (masked) hipLaunchKernelGGL((chunk_prep_kernel<true, 0, true>), grid, dim3(256), 0, st, p);
-      else if (cv == 0) hipLaunchKernelGGL((chunk_prep_kernel<true, 0, false>), grid, dim3(256), 0, st, p);
-      else if (cv == 1) hipLaunchKernelGGL((chunk_prep_kernel<true, 1, false>), grid, dim3(256), 0, st, p);
-      else hipLaunchKernelGGL((chunk_prep_kernel<true, 2, false>), grid, dim3(256), 0, st, p);
-    } else {
-      if (masked) hipLaunchKernelGGL((chunk_prep_kernel<false, 0, true>), grid, dim3(256), 0, st, p);
-      else if (cv == 0) hipLaunchKernelGGL((chunk_prep_kernel<false, 0, false>), grid, dim3(256), 0, st, p);
-      else if (cv == 1) hipLaunchKernelGGL((chunk_prep_kernel<false, 1, false>), grid, dim3(256), 0, st, p);
-      else hipLaunchKernelGGL((chunk_prep_kernel<false, 2, false>), grid, dim3(256), 0, st, p);
-    }
+    auto launch = [&](auto nh) {
+      constexpr int NH = decltype(nh)::value;
+      const dim3 grid(static_cast<unsigned>(chunks * (Hv / NH) + (p.order != nullptr ? 1 : 0))), block(256 * NH);
+      if (kt_lds) {
+        if (mask != nullptr) hipLaunchKernelGGL((chunk_prep_kernel<true, 0, true, NH>), grid, block, 0, st, p);
+        else if (cv == 0) hipLaunchKernelGGL((chunk_prep_kernel<true, 0, false, NH>), grid, block, 0, st, p);
+        else if (cv == 1) hipLaunchKernelGGL((chunk_prep_kernel<true, 1, false, NH>), grid, block, 0, st, p);
+        else hipLaunchKernelGGL((chunk_prep_kernel<true, 2, false, NH>), grid, block, 0, st, p);
+      } else {
+        if (mask != nullptr) hipLaunchKernelGGL((chunk_prep_kernel<false, 0, true, NH>), grid, block, 0, st, p);
+        else if (cv == 0) hipLaunchKernelGGL((chunk_prep_kernel<false, 0, false, NH>), grid, block, 0, st, p);
+        else if (cv == 1) hipLaunchKernelGGL((chunk_prep_kernel<false, 1, false, NH>), grid, block, 0, st, p);
+        else hipLaunchKernelGGL((chunk_prep_kernel<false, 2, false, NH>), grid, block, 0, st, p);
+      }
+    };
+    // Pairs where they leave the busiest CU no more heads than single ones do
+    // (us, prep and scan of Hv = 32 with the conv fused, single / pairs: 512
+    // tokens 33.2 / 35.0, 700 41.1 / 38.8, 1024 46.6 / 44.2, 1500 61.2 / 61.8,
+    // 2048 76.8 / 74.2, 4096 147.3 / 144.6; masked, two rows of 1000 58.4 /
+    // 56.6, four of 301 41.1 / 42.0).  Packed sequences stay single: their prep
+    // is bound by its writes (1024, 2560 and 7168 tokens 289.5 / 294).
+    const int64_t heads = chunks * Hv;
+    if (p.group % 2 == 0 && !packed && (heads / 2 + kCUs - 1) / kCUs * 2 <= (heads + kCUs - 1) / kCUs)
+      launch(std::integral_constant<int, 2>{});
+    else launch(std::integral_constant<int, 1>{});
     const int rc = gdn_host::check_launch("gdn_chunk_fwd/prep");
     if (rc != GDN_OK) return rc;
   }

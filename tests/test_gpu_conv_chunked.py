@@ -106,6 +106,21 @@ def test_rows_with_a_partial_chunk_equal_unfused(Hk, Hv, w_dtype):
     _assert_equal(_fused(t, Hk, Hv), _unfused(t, Hk, Hv))
 
 
+@pytest.mark.parametrize("Hk,Hv,w_dtype", [(16, 32, torch.bfloat16), (16, 32, torch.float32), (8, 32, torch.bfloat16)])
+def test_head_pairs_equal_single_heads(Hk, Hv, w_dtype):
+    """737 tokens of 32 heads take two v-heads a prep workgroup; the same rows as one packed sequence take
+    one.  The same arithmetic per head, so the same bits, fused and from q, k and v with and without a mask."""
+    T = 737
+    t = _inputs(2003 + Hk, 1, T, Hk, Hv, w_dtype=w_dtype)
+    _assert_equal(_fused(t, Hk, Hv), _fused(t, Hk, Hv, cu=[0, T]))
+    q, k, v, _ = mx.gdn_conv_prologue(t["qkv"], t["w"], Hk, Hv, D, D, t["cs"])
+    mask = torch.rand(1, T, generator=torch.Generator().manual_seed(5)) < 0.8
+    for m in (None, mask.to(DEV)):
+        args = (q, k, v, t["a"], t["b"], t["A_log"], t["dt_bias"], t["state"], m)
+        for x, y in zip(mx.gated_delta_update(*args), mx.gated_delta_update(*args, cu_seqlens=[0, T])):
+            assert torch.equal(x, y)
+
+
 @pytest.mark.parametrize("with_cs", [True, False])
 def test_packed_short_and_empty_sequences_equal_unfused(with_cs):
     """Lengths 2, 0, 68, 130, 1, 3: conv windows reaching into the conv
