@@ -287,6 +287,18 @@ int gdn_conv_prologue(const void* qkv, int io_dtype, int64_t qkv_stride, const v
                       int64_t B, int64_t S, int64_t Hk, int64_t Hv, int64_t Dk,
                       int64_t Dv, int64_t Kt, float eps, void* stream);
 
+/* Decode of the mixer from its mixed projection in one launch: the result of
+ * gdn_conv_prologue on one token per row (no mask) followed by the recurrent
+ * step with raw gates, bit for bit, without writing q, k and v.  bf16 qkv, taps
+ * and gates, A_log and dt_bias fp32 or bf16, Dk = Dv = 128.  conv_state_out
+ * (NULL: not wanted) must not alias conv_state_in (NULL: zeros); state_out may
+ * alias state_in (NULL: zeros).  y [B, Hv, Dv] bf16. */
+int gdn_conv_decode(const void* qkv, int64_t qkv_stride, const void* conv_w, const void* conv_state_in,
+                    void* conv_state_out, float eps, const void* a, const void* b, int64_t gate_stride,
+                    const void* A_log, const void* dt_bias, int param_dtype, const float* state_in,
+                    void* y, float* state_out, int64_t B, int64_t Hk, int64_t Hv, int64_t Dk, int64_t Dv,
+                    void* stream);
+
 /*
  * Conv-state commit of a partially accepted verify (dflash.py:424-425):
  * conv_state_out[b] = concat(conv_state_in[b], masked qkv[b])[n : n+Kt-1]

@@ -15,7 +15,7 @@ from typing import Optional
 import torch
 
 from . import _lib
-from .gated_delta import (CHUNK, IntSeq, PreparedCall, _contig, _cu_seqlens, _dtype_code, _gate_codes, _gate_pair,
+from .gated_delta import (CHUNK, IntSeq, PreparedCall, _addr, _contig, _cu_seqlens, _dtype_code, _gate_codes, _gate_pair,
                           _int_rows, _mask_u8, _on_device, _param_codes, _ptr, _require_device, _state_operands, _stream,
                           _token_rows)
 
@@ -242,6 +242,55 @@ def gdn_conv_chunked(qkv: torch.Tensor, conv_weight: torch.Tensor, num_k_heads: 
     with _on_device(dev):
         _lib.call("gdn_chunk_fwd_conv", *args)
     return outs
+
+
+CONV_DECODE_MAX_ROWS = 64  # where one launch is no slower than two (conv_decode_kernel's figures)
+
+
+def gdn_conv_decode(qkv, conv_weight, num_k_heads, num_v_heads, head_k_dim, head_v_dim, a, b, A_log, dt_bias, state,
+                    conv_state, *, eps: float = 1e-6, write_conv_state: bool = True):
+    """A decode step of the mixer from its mixed projection in one launch
+    (``gdn_conv_decode``): :func:`gdn_conv_prologue` on one token per row, then
+    ``gated_delta_update``, bit for bit.  Arguments as there; dense states.
+
+    Returns ``(y, new_state, new_conv_state)``, or None for operands it does
+    not take (other types, head sizes, taps or layouts, more than 64 rows):
+    the caller then runs the two, which check them.
+    """
+    B, S, C = qkv.shape
+    Hk, Hv, D = num_k_heads, num_v_heads, 128
+    bf16 = torch.bfloat16
+    if (S != 1 or not 1 <= B <= CONV_DECODE_MAX_ROWS or head_k_dim != D or head_v_dim != D
+            or C != 2 * Hk * D + Hv * D or Hv % Hk != 0 or Hv > 65535
+            or qkv.dtype is not bf16 or a.dtype is not bf16 or b.dtype is not bf16
+            or conv_weight.dtype is not bf16 or conv_weight.shape != (C, 4) or not conv_weight.is_contiguous()
+            or a.shape != (B, 1, Hv) or b.shape != (B, 1, Hv) or A_log.shape != (Hv,) or dt_bias.shape != (Hv,)
+            or A_log.dtype is not dt_bias.dtype or A_log.dtype not in (torch.float32, bf16)
+            or not A_log.is_contiguous() or not dt_bias.is_contiguous()):
+        return None
+    if state is not None and (state.dtype is not torch.float32 or state.shape != (B, Hv, D, D)
+                              or not state.is_contiguous()):
+        return None
+    if conv_state is not None and (conv_state.dtype is not bf16 or conv_state.shape != (B, 3, C)
+                                   or not conv_state.is_contiguous()):
+        return None
+    ld, la = _token_rows(qkv, C), _token_rows(a, Hv)
+    if ld is None or ld % 8 != 0 or la is None or la != _token_rows(b, Hv):
+        return None
+    qkv_p, w_p = qkv.data_ptr(), conv_weight.data_ptr()
+    st_p, cs_p = _addr(state), _addr(conv_state)
+    if (qkv_p | w_p | st_p | cs_p) % 16 != 0:
+        return None
+    dev = _require_device((qkv, conv_weight, a, b, A_log, dt_bias, state, conv_state),
+                          ("qkv", "conv_weight", "a", "b", "A_log", "dt_bias", "state", "conv_state"))
+    y = torch.empty(B, 1, Hv, D, dtype=bf16, device=dev)
+    new_state = torch.empty(B, Hv, D, D, dtype=torch.float32, device=dev)
+    cs_out = torch.empty(B, 3, C, dtype=bf16, device=dev) if write_conv_state else None
+    with _on_device(dev):
+        _lib.call("gdn_conv_decode", qkv_p, ld, w_p, cs_p, _addr(cs_out), float(eps), a.data_ptr(), b.data_ptr(), la,
+                  A_log.data_ptr(), dt_bias.data_ptr(), _dtype_code(A_log, "A_log"), st_p, y.data_ptr(),
+                  new_state.data_ptr(), B, Hk, Hv, D, D, _stream(dev))
+    return y, new_state, cs_out
 
 
 def prepare_conv_chunked(qkv, conv_weight, num_k_heads, num_v_heads, head_k_dim, head_v_dim, a, b, A_log, dt_bias,

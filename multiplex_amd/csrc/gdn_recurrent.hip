@@ -356,6 +356,122 @@ __global__ __launch_bounds__(256) void recurrent_kernel(const RecParams p) {
   if (write_state && commit == 1 && row_ok) store_row<4, LPR>(p.state_out + static_cast<size_t>(srow) * DK, sub, s);
 }
 
+// Decode from the mixed projection: the conv prologue (prologue_kernel in
+// gdn_prologue.hip) and the recurrence of one token per row in one launch, for
+// bf16 rows and taps at 128-wide heads.  A workgroup takes 8 U state rows of a
+// (row, v-head).  Its first wave forms the head's q, k and v with the
+// prologue's arithmetic -- 16 lanes a head, 8 channels a lane -- while every
+// wave's state rows are on their way, and passes them through LDS (rounded to
+// bf16, as the prologue's outputs are); then the state steps as in
+// recurrent_kernel, so y, state and conv state are the two launches' bits.
+// The state stream bounds it; the conv, repeated by each of a head's 16 / U
+// workgroups, hides behind it where the two launches ran one after the other,
+// with q, k and v through memory between them.  Graph-replayed at Hv = 32, the
+// two launches against U = 2 / 4 / 8 (us): 1 row 5.6, 3.8 / 4.1 / 4.6; 4 rows
+// 7.3, 5.4 / 5.1 / 5.4; 8 rows 10.0, 8.0 / 7.9 / 6.9 (4.9 TB/s); 16 rows 15.1,
+// 14.6 / 14.0 / 12.9; 64 rows 47.8, 50.6 / 48.1 / 47.5.
+struct ConvDecodeParams {
+  const uint16_t* qkv;  // [B] rows of C = 2 Hk 128 + Hv 128 channels, ld apart
+  int64_t ld;
+  const uint16_t* w;    // [C][4] taps
+  const uint16_t* cs_in;  // [B][3][C] or null (zeros)
+  uint16_t* cs_out;       // [B][3][C] or null; not cs_in
+  const float* state_in;  // [B][Hv][128][128] or null (zeros)
+  float* state_out;
+  uint16_t* y;            // [B][Hv][128]
+  GateArgs ga;
+  int Hk, Hv, group, C;
+  float eps;
+};
+
+template <int GF, int U>
+__global__ __launch_bounds__(256) void conv_decode_kernel(const ConvDecodeParams p) {
+  constexpr int D = 128, LPR = D / 4, DT = GDN_DTYPE_BF16;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int sub = lane & (LPR - 1);
+  const int64_t row = blockIdx.z;
+  const int hv = blockIdx.y, hk = hv / p.group;
+  __shared__ __align__(16) float qkvs[3][D];
+
+  // the first wave's conv operands: role 0 = q, 1 = k, 2 = v (the last 16 lanes repeat v's and store nothing)
+  const int role = min(lane >> 4, 2);
+  const int ch = 8 * (lane & 15);
+  const int c0 = (role == 0 ? hk : role == 1 ? p.Hk + hk : 2 * p.Hk + hv) * D + ch;
+  Raw8<DT> wr[4], xw[3], x;
+  if (wave == 0) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) wr[i] = load_raw8<DT>(p.w, static_cast<int64_t>(c0) * 4 + 8 * i);
+    // without a conv state the rows are zeros: the qkv row stands in for the loads
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+      xw[i] = load_raw8<DT>(p.cs_in != nullptr ? p.cs_in : p.qkv,
+                            p.cs_in != nullptr ? (row * 3 + i) * p.C + c0 : row * p.ld + c0);
+    x = load_raw8<DT>(p.qkv, row * p.ld + c0);
+  }
+  float al, db, gx, gy;
+  param_load_raw<GF, DT>(p.ga, hv, al, db);
+  gate_load<GF, DT>(p.ga, row * p.ga.ld + hv, gx, gy);
+
+  // unit u of a wave: state rows dv0 + 2 u, + 1 (32 lanes each, one float4 a lane)
+  const int dv0 = (static_cast<int>(blockIdx.x) * 4 + wave) * 2 * U + (lane >> 5);
+  const int64_t srow0 = ((row * p.Hv + hv) * D + dv0) * D;
+  float s[U][4];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const float* src = p.state_in != nullptr ? p.state_in + srow0 + 2 * u * D : kZeroRow;
+    const f32x4 v = __builtin_nontemporal_load((gbl_f32x4*)(src + sub * 4));
+#pragma unroll
+    for (int e = 0; e < 4; ++e) s[u][e] = v[e];
+  }
+  __builtin_amdgcn_sched_barrier(0);  // every load is issued before the first wait
+
+  if (wave == 0) {
+    const bool has_cs = p.cs_in != nullptr;
+    u32x4 rw[3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) rw[i] = row_or_zero(has_cs, xw[i].v);
+    uint32_t pa[CPL], pc[CPL];  // p(t - 2), p(t)
+    row_pairs(rw[0], rw[1], pa);
+    row_pairs(rw[2], x.v, pc);
+    float o[CPL], ss = 0.0f;
+#pragma unroll
+    for (int j = 0; j < CPL; ++j) {
+      o[j] = silu(conv_pairs(wr[j >> 1].v[2 * (j & 1)], wr[j >> 1].v[2 * (j & 1) + 1], pa[j], pc[j]));
+      ss = fmaf(o[j], o[j], ss);
+    }
+    ss = head_sum<16>(ss);
+    const float post = role == 0 ? 1.0f / static_cast<float>(D) : rsqrtf(static_cast<float>(D));
+    const float sc = role == 2 ? 1.0f : rsqrtf(ss / static_cast<float>(D) + p.eps) * post;
+#pragma unroll
+    for (int j = 0; j < CPL; ++j) o[j] = bf16_to_f32(f32_to_bf16(o[j] * sc));
+    *reinterpret_cast<f32x4*>(&qkvs[role][ch]) = f32x4{o[0], o[1], o[2], o[3]};
+    *reinterpret_cast<f32x4*>(&qkvs[role][ch + 4]) = f32x4{o[4], o[5], o[6], o[7]};
+    // the new conv state, once per channel: v's by the head's first workgroup, q's and k's by that of the
+    // k-head's first v-head
+    if (p.cs_out != nullptr && blockIdx.x == 0 && lane < 48 && (role == 2 || hv % p.group == 0)) {
+      uint16_t* dst = p.cs_out + row * 3 * p.C + c0;
+      *reinterpret_cast<u32x4*>(dst) = rw[1];
+      *reinterpret_cast<u32x4*>(dst + p.C) = rw[2];
+      *reinterpret_cast<u32x4*>(dst + 2 * static_cast<int64_t>(p.C)) = x.v;
+    }
+  }
+  __syncthreads();
+
+  const f32x4 q4 = *reinterpret_cast<const f32x4*>(&qkvs[0][4 * sub]);
+  const f32x4 k4 = *reinterpret_cast<const f32x4*>(&qkvs[1][4 * sub]);
+  const float qf[4] = {q4.x, q4.y, q4.z, q4.w}, kf[4] = {k4.x, k4.y, k4.z, k4.w};
+  float g, beta;
+  gate_transform<GF>(GDN_GATES_RAW, gx, gy, exp_fast(al), db, g, beta);
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    step_row<4, LPR>(s[u], kf, qkvs[2][dv0 + 2 * u], g, beta);
+    const float yv = row_dot<4, LPR>(s[u], qf);
+    if (sub == 0) p.y[(row * p.Hv + hv) * D + dv0 + 2 * u] = f32_to_bf16(yv);
+    store_row<4, LPR>(p.state_out + srow0 + 2 * u * D, sub, s[u]);
+  }
+}
+
 // Multi-token body (verify, commit, packed rows): the workgroup (always 4
 // waves, 32 state rows) stages a tile of TILE tokens -- k and q as fp32, the
 // transformed gates, the mask and the v values of its rows -- in LDS, then
@@ -1195,4 +1311,68 @@ extern "C" int gdn_gated_delta_kernel(const void* q, const void* k, const void* 
   r.Dv = Dv;
   r.stream = stream;
   return run_recurrent(&r);
+}
+
+extern "C" int gdn_conv_decode(const void* qkv, int64_t qkv_stride, const void* conv_w, const void* conv_state_in,
+                               void* conv_state_out, float eps, const void* a, const void* b, int64_t gate_stride,
+                               const void* A_log, const void* dt_bias, int param_dtype, const float* state_in,
+                               void* y, float* state_out, int64_t B, int64_t Hk, int64_t Hv, int64_t Dk, int64_t Dv,
+                               void* stream) {
+  using gdn_host::fail;
+  if (Dk != 128 || Dv != 128)
+    return fail(GDN_ERR_UNSUPPORTED, "gdn_conv_decode: built for Dk = Dv = 128 (got %lld, %lld)", (long long)Dk,
+                (long long)Dv);
+  if (B < 0 || Hk <= 0 || Hv <= 0 || Hv % Hk != 0 || B > 65535 || Hv > 65535)
+    return fail(GDN_ERR_INVALID, "gdn_conv_decode: bad sizes");
+  if (param_dtype != GDN_DTYPE_F32 && param_dtype != GDN_DTYPE_BF16)
+    return fail(GDN_ERR_UNSUPPORTED, "gdn_conv_decode: A_log and dt_bias must be fp32 or bf16");
+  if (!(eps >= 0.0f)) return fail(GDN_ERR_INVALID, "gdn_conv_decode: eps must be >= 0");
+  const int64_t C = 2 * Hk * Dk + Hv * Dv;
+  if ((qkv_stride != 0 && (qkv_stride < C || qkv_stride % 8 != 0)) || (gate_stride != 0 && gate_stride < Hv))
+    return fail(GDN_ERR_INVALID, "gdn_conv_decode: strides must cover the rows (qkv's a multiple of 8)");
+  if (B == 0) return GDN_OK;
+  if (!qkv || !conv_w || !a || !b || !A_log || !dt_bias || !y || !state_out)
+    return fail(GDN_ERR_INVALID, "gdn_conv_decode: null pointer");
+  if (conv_state_out != nullptr && conv_state_out == conv_state_in)
+    return fail(GDN_ERR_INVALID, "gdn_conv_decode: conv_state_out must not alias conv_state_in");
+  if (!gdn_host::aligned(qkv, 16) || !gdn_host::aligned(conv_w, 16) || !gdn_host::aligned(conv_state_in, 16) ||
+      !gdn_host::aligned(conv_state_out, 16) || !gdn_host::aligned(state_in, 16) || !gdn_host::aligned(state_out, 16))
+    return fail(GDN_ERR_INVALID, "gdn_conv_decode: misaligned pointer");
+  ConvDecodeParams p;
+  p.qkv = static_cast<const uint16_t*>(qkv);
+  p.ld = qkv_stride > 0 ? qkv_stride : C;
+  p.w = static_cast<const uint16_t*>(conv_w);
+  p.cs_in = static_cast<const uint16_t*>(conv_state_in);
+  p.cs_out = static_cast<uint16_t*>(conv_state_out);
+  p.state_in = state_in;
+  p.state_out = state_out;
+  p.y = static_cast<uint16_t*>(y);
+  p.ga.gx = a;
+  p.ga.gy = b;
+  p.ga.A_log = A_log;
+  p.ga.dt_bias = dt_bias;
+  p.ga.ld = gate_stride > 0 ? gate_stride : Hv;
+  p.ga.mode = GDN_GATES_RAW;
+  p.ga.gdt = GDN_DTYPE_BF16;
+  p.ga.pdt = param_dtype;
+  p.Hk = static_cast<int>(Hk);
+  p.Hv = static_cast<int>(Hv);
+  p.group = static_cast<int>(Hv / Hk);
+  p.C = static_cast<int>(C);
+  p.eps = eps;
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  auto launch = [&](auto unit) {
+    constexpr int U = decltype(unit)::value;
+    const dim3 grid(16 / U, static_cast<unsigned>(Hv), static_cast<unsigned>(B));
+    if (param_dtype == GDN_DTYPE_F32)
+      hipLaunchKernelGGL((conv_decode_kernel<GF_IO_F32, U>), grid, dim3(256), 0, st, p);
+    else
+      hipLaunchKernelGGL((conv_decode_kernel<GF_IO_IO, U>), grid, dim3(256), 0, st, p);
+  };
+  // more state rows a workgroup (fewer repeats of the conv) as the heads fill the CUs by themselves
+  // (conv_decode_kernel's comment has both sides)
+  if (B * Hv < 128) launch(std::integral_constant<int, 2>{});
+  else if (B * Hv < 256) launch(std::integral_constant<int, 4>{});
+  else launch(std::integral_constant<int, 8>{});
+  return gdn_host::check_launch("gdn_conv_decode");
 }

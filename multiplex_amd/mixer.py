@@ -18,7 +18,9 @@ Data path per call:
   gated_delta_update           recurrent or chunked kernel (HIP); where the
                                chunked kernel runs (long unmasked rows) the
                                prologue is fused into its prep instead
-                               (``gdn_conv_chunked``)
+                               (``gdn_conv_chunked``), and for one token per
+                               unmasked row of dense states into the recurrent
+                               step (``gdn_conv_decode``)
   norm(out, z) + out_proj      up to 16 rows (decode of up to 16 rows) one
                                ``gdn_linear_decode`` launch with the gated
                                RMSNorm in its operand load (HIP); else the
@@ -42,7 +44,7 @@ from typing import Optional, Sequence
 import torch
 
 from .cache import ArraysCache
-from .conv import conv_state_commit, gdn_conv_chunked, gdn_conv_prologue
+from .conv import conv_state_commit, gdn_conv_chunked, gdn_conv_decode, gdn_conv_prologue
 from .epilogue import gated_rms_norm
 from .state_pool import PooledBatch
 from .gated_delta import CHUNK_MIN_TOKENS, IntSeq, gated_delta_commit, gated_delta_update, gated_delta_verify
@@ -208,6 +210,16 @@ class GatedDeltaNet(torch.nn.Module):
                 if not pooled:
                     cache[1] = new_state
             return self._epilogue(y, z)
+        if mask is None and not verify and not pooled and qkv.shape[1] == 1:
+            # decode on dense states: the conv prologue and the step in one launch (bit-identical to the two below)
+            step = gdn_conv_decode(qkv, self.conv1d_weight, self.num_k_heads, self.num_v_heads, self.head_k_dim,
+                                   self.head_v_dim, a, b, self.A_log, self.dt_bias, state, conv_state,
+                                   eps=self.rms_norm_eps, write_conv_state=cache is not None)
+            if step is not None:
+                y, new_state, new_cs = step
+                if cache is not None:
+                    cache[0], cache[1] = new_cs, new_state
+                return self._epilogue(y, z)
         # pooled decode advances the conv state in place too, as its states
         # advance in their pool slots (no new tensor per step)
         cs_in_place = (pooled and not verify and qkv.shape[1] == 1 and conv_state is not None
