@@ -236,6 +236,22 @@ int gdn_chunk_fwd_conv(const void* qkv, int64_t qkv_stride, const void* conv_w,
                        int64_t chunk, void* workspace, size_t workspace_bytes,
                        void* stream);
 
+/* gdn_chunk_fwd_conv with a token mask [n_tok] (0 = masked; NULL: none), as
+ * gdn_conv_prologue and gdn_chunk_fwd take one: a masked token's qkv row is zeros
+ * to the conv (and to the new conv state), it keeps the state and its y is 0. */
+int gdn_chunk_fwd_conv_masked(const void* qkv, int64_t qkv_stride, const void* conv_w,
+                       int conv_w_dtype, const void* conv_state_in,
+                       void* conv_state_out, float eps, int gate_mode,
+                       const void* gx, const void* gy, int gate_dtype,
+                       int64_t gate_stride, const void* A_log,
+                       const void* dt_bias, int param_dtype,
+                       const uint8_t* mask, const float* state_in, void* y, float* state_out,
+                       const int32_t* state_index, int64_t n_slots,
+                       const int32_t* cu_seqlens, int64_t n_seqs, int64_t n_tok,
+                       int64_t Hk, int64_t Hv, int64_t Dk, int64_t Dv,
+                       int64_t chunk, void* workspace, size_t workspace_bytes,
+                       void* stream);
+
 /*
  * gdn_chunk_fwd without a workspace argument: the chunk records go to a
  * static device array of 64 MiB (67,108,864 bytes) inside the library,

@@ -42,6 +42,7 @@ EXPORTS = (
     "gdn_chunk_fwd_noalloc",
     "gdn_chunk_conv_workspace_bytes",
     "gdn_chunk_fwd_conv",
+    "gdn_chunk_fwd_conv_masked",
     "gdn_conv_decode",
     "gdn_conv_prologue",
     "gdn_conv_state_commit",
@@ -154,6 +155,11 @@ _SIGNATURES = {
     "gdn_chunk_fwd_conv": (
         c_int,
         [_P, _I64, _P, c_int, _P, _P, c_float, c_int, _P, _P, c_int, _I64, _P, _P, c_int, _P, _P, _P, _P, _I64, _P,
+         _I64, _I64, _I64, _I64, _I64, _I64, _I64, _P, c_size_t, _P],
+    ),
+    "gdn_chunk_fwd_conv_masked": (
+        c_int,
+        [_P, _I64, _P, c_int, _P, _P, c_float, c_int, _P, _P, c_int, _I64, _P, _P, c_int, _P, _P, _P, _P, _P, _I64, _P,
          _I64, _I64, _I64, _I64, _I64, _I64, _I64, _P, c_size_t, _P],
     ),
     "gdn_conv_decode": (

@@ -170,9 +170,11 @@ def conv_chunk_workspace_bytes(n_seqs: int, n_tok: int, Hv: int, Dk: int, Dv: in
 
 
 def _conv_chunked_args(qkv, conv_weight, num_k_heads, num_v_heads, head_k_dim, head_v_dim, a, b, A_log, dt_bias,
-                       state, conv_state, cu_seqlens, eps, state_out, workspace, state_index, write_conv_state):
-    dev = _require_device([qkv, conv_weight, a, b, A_log, dt_bias, state, conv_state, state_out],
-                          ["qkv", "conv_weight", "a", "b", "A_log", "dt_bias", "state", "conv_state", "state_out"])
+                       state, conv_state, cu_seqlens, eps, state_out, workspace, state_index, write_conv_state,
+                       mask=None):
+    dev = _require_device([qkv, conv_weight, a, b, A_log, dt_bias, state, conv_state, state_out, mask],
+                          ["qkv", "conv_weight", "a", "b", "A_log", "dt_bias", "state", "conv_state", "state_out",
+                           "mask"])
     if qkv.dim() != 3 or qkv.dtype != torch.bfloat16:
         raise ValueError("qkv must be [B, S, C] bf16")
     B, S, C = qkv.shape
@@ -202,6 +204,7 @@ def _conv_chunked_args(qkv, conv_weight, num_k_heads, num_v_heads, head_k_dim, h
     gate_code = _gate_codes(gx, gy)
     param_code = _param_codes(A_log, dt_bias, Hv)
     A_log, dt_bias = _contig(A_log), _contig(dt_bias)
+    mask_u8 = _mask_u8(mask, (B, S))
     n_tok = B * S
     state, out_state, idx, n_slots = _state_operands(state, state_out, True, n_seqs, Hv, Dv, Dk, dev, state_index)
     y = torch.empty(B, S, Hv, Dv, dtype=qkv.dtype, device=dev)
@@ -210,10 +213,10 @@ def _conv_chunked_args(qkv, conv_weight, num_k_heads, num_v_heads, head_k_dim, h
     if workspace is None or workspace.numel() * workspace.element_size() < ws_bytes:
         workspace = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=dev)
     args = (_ptr(qkv), ld, _ptr(w), wdt, _ptr(conv_state), _ptr(cs_out), float(eps), _lib.GATES_RAW, _ptr(gx),
-            _ptr(gy), gate_code, g_ld, _ptr(A_log), _ptr(dt_bias), param_code, _ptr(state), _ptr(y), _ptr(out_state),
-            _ptr(idx), n_slots, _ptr(cu), n_seqs, n_tok, Hk, Hv, Dk, Dv, CHUNK, _ptr(workspace), ws_bytes,
-            _stream(dev))
-    keep = dict(qkv=qkv, w=w, conv_state=conv_state, gx=gx, gy=gy, A_log=A_log, dt_bias=dt_bias, state=state,
+            _ptr(gy), gate_code, g_ld, _ptr(A_log), _ptr(dt_bias), param_code, _ptr(mask_u8), _ptr(state), _ptr(y),
+            _ptr(out_state), _ptr(idx), n_slots, _ptr(cu), n_seqs, n_tok, Hk, Hv, Dk, Dv, CHUNK, _ptr(workspace),
+            ws_bytes, _stream(dev))
+    keep = dict(qkv=qkv, w=w, mask=mask_u8, conv_state=conv_state, gx=gx, gy=gy, A_log=A_log, dt_bias=dt_bias, state=state,
                 cu=cu, workspace=workspace, state_index=idx, y=y, state_out=out_state, cs_out=cs_out)
     return args, keep, (y, out_state, cs_out), dev
 
@@ -223,7 +226,7 @@ def gdn_conv_chunked(qkv: torch.Tensor, conv_weight: torch.Tensor, num_k_heads: 
                      dt_bias: torch.Tensor, state: Optional[torch.Tensor] = None,
                      conv_state: Optional[torch.Tensor] = None, *, cu_seqlens: Optional[IntSeq] = None,
                      eps: float = 1e-6, state_out: Optional[torch.Tensor] = None, workspace=None,
-                     state_index=None, write_conv_state: bool = True):
+                     state_index=None, write_conv_state: bool = True, mask: Optional[torch.Tensor] = None):
     """The prefill of the mixer from its mixed projection: the conv prologue
     (``dflash.py:351-370``) fused into the chunked pass's prep
     (``gdn_chunk_fwd_conv``), then the chunked gated delta rule
@@ -232,15 +235,15 @@ def gdn_conv_chunked(qkv: torch.Tensor, conv_weight: torch.Tensor, num_k_heads: 
     Equal bit for bit to :func:`gdn_conv_prologue` followed by
     ``gated_delta_update(..., chunked=True)``, without writing q, k and v
     (only v, into the workspace, for the scan).  qkv ``[B, S, C]`` bf16 (or a
-    one-stride column slice of a fused in_proj output), no mask; a, b
-    ``[B, S, Hv]``; Dk = Dv = 128; other arguments as in those two
-    functions.
+    one-stride column slice of a fused in_proj output); mask ``[B, S]`` or
+    None; a, b ``[B, S, Hv]``; Dk = Dv = 128; other arguments as in those
+    two functions.
     """
     args, _keep, outs, dev = _conv_chunked_args(qkv, conv_weight, num_k_heads, num_v_heads, head_k_dim,
                                                 head_v_dim, a, b, A_log, dt_bias, state, conv_state, cu_seqlens,
-                                                eps, state_out, workspace, state_index, write_conv_state)
+                                                eps, state_out, workspace, state_index, write_conv_state, mask)
     with _on_device(dev):
-        _lib.call("gdn_chunk_fwd_conv", *args)
+        _lib.call("gdn_chunk_fwd_conv_masked", *args)
     return outs
 
 
@@ -306,4 +309,4 @@ def prepare_conv_chunked(qkv, conv_weight, num_k_heads, num_v_heads, head_k_dim,
     for name, given in (("qkv", qkv), ("gx", a), ("gy", b)):
         if keep[name].data_ptr() != given.data_ptr():
             raise ValueError(f"{name} must be contiguous or a one-stride column slice for a prepared launch")
-    return PreparedCall("gdn_chunk_fwd_conv", args, keep, outs, dev)
+    return PreparedCall("gdn_chunk_fwd_conv_masked", args, keep, outs, dev)

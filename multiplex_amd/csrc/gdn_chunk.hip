@@ -285,8 +285,9 @@ constexpr int KTAP = 4;  // conv taps
 // lanes, in the prologue's lane order).  x runs over X = the sequence's conv
 // state (3 rows; zeros without one) followed by its qkv rows.  Tokens past
 // the chunk's end repeat its last row.  Every load is issued before the
-// first conversion.
-template <int WDT, int R, bool NORM>
+// first conversion.  MASK: a masked token's qkv row is zeros (a select, as the
+// prologue's).
+template <int WDT, int R, bool NORM, bool MASK>
 __device__ __forceinline__ void conv_run(const ChunkParams& p, const ChunkPos& cp, int c0, int t0, float post,
                                          u32x4 (&out)[R]) {
   Raw8<WDT> wr[KTAP];
@@ -308,11 +309,19 @@ __device__ __forceinline__ void conv_run(const ChunkParams& p, const ChunkPos& c
                                : (cp.seq_tok0 + tp) * p.qkv_ld + c0;
     xw[i] = load_raw8<GDN_DTYPE_BF16>(cs_row ? static_cast<const void*>(p.cs_in) : p.qkv, off);
     wm[i] = from_cs && !cs_row ? 0.0f : 1.0f;
+    if constexpr (MASK) {
+      const uint8_t on = *(gbl_u8*)(p.mask + cp.seq_tok0 + tp);
+      wm[i] = from_cs || on != 0 ? wm[i] : 0.0f;
+    }
   }
   Raw8<GDN_DTYPE_BF16> xs[R];
+  uint8_t xm[R];
 #pragma unroll
-  for (int u = 0; u < R; ++u)
-    xs[u] = load_raw8<GDN_DTYPE_BF16>(p.qkv, (cp.tok0 + min(t0 + u, cp.len - 1)) * p.qkv_ld + c0);
+  for (int u = 0; u < R; ++u) {
+    const int64_t tok = cp.tok0 + min(t0 + u, cp.len - 1);
+    xs[u] = load_raw8<GDN_DTYPE_BF16>(p.qkv, tok * p.qkv_ld + c0);
+    xm[u] = MASK ? *(gbl_u8*)(p.mask + tok) : 1;
+  }
   // token u's SiLU outputs o and their sum of squares ss -> out[u]
   auto finish = [&](int u, float (&o)[CPL], float ss) {
     if constexpr (NORM) {
@@ -338,8 +347,9 @@ __device__ __forceinline__ void conv_run(const ChunkParams& p, const ChunkPos& c
     row_pairs(rw[1], rw[2], pb);
 #pragma unroll
     for (int u = 0; u < R; ++u) {
+      const u32x4 xr = MASK ? row_or_zero(xm[u] != 0, xs[u].v) : xs[u].v;
       uint32_t pc[CPL];  // p(t)
-      row_pairs(rw[KTAP - 2], xs[u].v, pc);
+      row_pairs(rw[KTAP - 2], xr, pc);
       float o[CPL];
       float ss = 0.0f;
 #pragma unroll
@@ -352,7 +362,7 @@ __device__ __forceinline__ void conv_run(const ChunkParams& p, const ChunkPos& c
         pa[j] = pb[j];
         pb[j] = pc[j];
       }
-      rw[KTAP - 2] = xs[u].v;
+      rw[KTAP - 2] = xr;
       finish(u, o, ss);
     }
   } else {
@@ -380,6 +390,7 @@ __device__ __forceinline__ void conv_run(const ChunkParams& p, const ChunkPos& c
       float ss = 0.0f;
 #pragma unroll
       for (int j = 0; j < CPL; ++j) {
+        if constexpr (MASK) x[j] = xm[u] != 0 ? x[j] : 0.0f;
         float acc = w[KTAP - 1][j] * x[j];
 #pragma unroll
         for (int i = 0; i < KTAP - 1; ++i) acc = fmaf(w[i][j], win[i][j], acc);
@@ -401,6 +412,7 @@ __device__ __forceinline__ void conv_run(const ChunkParams& p, const ChunkPos& c
 // (or of an empty sequence): X's last 3 rows, X[len + i], on the channels
 // of this v-head and, from the k-head's first v-head, of its q and k heads.
 // Thread i < 144 copies 8 channels of one row.
+template <bool MASK>
 __device__ __forceinline__ void conv_state_rows(const ChunkParams& p, int seq, int64_t seq_tok0, int seq_len,
                                                 int hk, int hv, bool first_v, int tid) {
   if (p.cs_out == nullptr || tid >= 3 * 48) return;
@@ -411,7 +423,9 @@ __device__ __forceinline__ void conv_state_rows(const ChunkParams& p, int seq, i
   const int xi = seq_len + row;
   u32x4 v = {0u, 0u, 0u, 0u};
   if (xi >= KTAP - 1) {
-    v = *reinterpret_cast<const u32x4*>(p.qkv + (seq_tok0 + xi - (KTAP - 1)) * p.qkv_ld + c0);
+    const int64_t tok = seq_tok0 + xi - (KTAP - 1);
+    v = *reinterpret_cast<const u32x4*>(p.qkv + tok * p.qkv_ld + c0);
+    if constexpr (MASK) v = row_or_zero(p.mask[tok] != 0, v);
   } else if (p.cs_in != nullptr) {
     v = *reinterpret_cast<const u32x4*>(p.cs_in + (static_cast<int64_t>(seq) * (KTAP - 1) + xi) * p.C + c0);
   }
@@ -497,7 +511,7 @@ __global__ __launch_bounds__(256 * NH) __attribute__((amdgpu_waves_per_eu(4))) v
   if (!chunk_at(p, c, cp)) {
     if constexpr (CONV != 0) {
       if (p.cu != nullptr && cp.seq_len == 0 && cp.ci == 0)
-        conv_state_rows(p, cp.seq, cp.seq_tok0, 0, hk, hv, first_v && hsel == 0, tid4);
+        conv_state_rows<MASK>(p, cp.seq, cp.seq_tok0, 0, hk, hv, first_v && hsel == 0, tid4);
     }
     return;
   }
@@ -587,11 +601,13 @@ __global__ __launch_bounds__(256 * NH) __attribute__((amdgpu_waves_per_eu(4))) v
       u32x4 o[RPT];
       const int t0 = RPT * (4 * wave + lq);
       const float post = role == 0 ? 1.0f / static_cast<float>(DK) : rsqrtf(static_cast<float>(DK));
-      conv_run<WDT, RPT, true>(p, cp, (role * p.Hk + hk) * DK + 8 * g, t0, post, o);
+      conv_run<WDT, RPT, true, MASK>(p, cp, (role * p.Hk + hk) * DK + 8 * g, t0, post, o);
 #pragma unroll
       for (int u = 0; u < RPT; ++u) {
         const int r = t0 + u;
-        const u32x4 val = row_or_zero(r < len, o[u]);
+        // (a masked token's q and k are zeros, as with CONV = 0)
+        const bool on = r < len && (!MASK || *(gbl_u8*)(p.mask + tok0 + min(r, len - 1)) != 0);
+        const u32x4 val = row_or_zero(on, o[u]);
         *reinterpret_cast<u32x4*>(role == 0 ? &Qs[r][8 * g] : &Ks[r][8 * g]) = val;
         if (first_v)
           *reinterpret_cast<u32x4*>(reinterpret_cast<uint16_t*>(rec_k + (role == 0 ? kOffQf : kOffKf)) +
@@ -601,14 +617,14 @@ __global__ __launch_bounds__(256 * NH) __attribute__((amdgpu_waves_per_eu(4))) v
     {
       u32x4 o[4];
       const int t0 = 4 * (4 * w4 + lq);
-      conv_run<WDT, 4, false>(p, cp, 2 * p.Hk * DK + hv * DV + 8 * g, t0, 1.0f, o);
+      conv_run<WDT, 4, false, MASK>(p, cp, 2 * p.Hk * DK + hv * DV + 8 * g, t0, 1.0f, o);
 #pragma unroll
       for (int u = 0; u < 4; ++u)
         if (t0 + u < len)
           *reinterpret_cast<u32x4*>(p.v_out + ((tok0 + t0 + u) * p.Hv + hv) * DV + 8 * g) = o[u];
     }
     if (cp.ci == n_chunks(cp.seq_len) - 1)
-      conv_state_rows(p, cp.seq, cp.seq_tok0, cp.seq_len, hk, hv, first_v && hsel == 0, tid4);
+      conv_state_rows<MASK>(p, cp.seq, cp.seq_tok0, cp.seq_len, hk, hv, first_v && hsel == 0, tid4);
   }
   __syncthreads();
 
@@ -1429,21 +1445,22 @@ int chunk_fwd(const void* q, const void* k, const void* v, int qkv_dtype, int ga
   const bool kt_lds = static_cast<int64_t>(kTiles) * n_seqs * Hv > kCUs;
   if ((phases & kPhasePrep) && chunks > 0) {
     // one workgroup per (chunk slot, v-head or pair of a k-head's), and one more that orders packed sequences
-    // (the fused prologue takes no mask: conv != null implies mask == null)
     const int cv = conv == nullptr ? 0 : (conv->w_dtype == GDN_DTYPE_F32 ? 2 : 1);
     auto launch = [&](auto nh) {
       constexpr int NH = decltype(nh)::value;
       const dim3 grid(static_cast<unsigned>(chunks * (Hv / NH) + (p.order != nullptr ? 1 : 0))), block(256 * NH);
+      auto prep = [&](auto kt, auto masked) {
+        constexpr bool K = decltype(kt)::value, M = decltype(masked)::value;
+        if (cv == 0) hipLaunchKernelGGL((chunk_prep_kernel<K, 0, M, NH>), grid, block, 0, st, p);
+        else if (cv == 1) hipLaunchKernelGGL((chunk_prep_kernel<K, 1, M, NH>), grid, block, 0, st, p);
+        else hipLaunchKernelGGL((chunk_prep_kernel<K, 2, M, NH>), grid, block, 0, st, p);
+      };
       if (kt_lds) {
-        if (mask != nullptr) hipLaunchKernelGGL((chunk_prep_kernel<true, 0, true, NH>), grid, block, 0, st, p);
-        else if (cv == 0) hipLaunchKernelGGL((chunk_prep_kernel<true, 0, false, NH>), grid, block, 0, st, p);
-        else if (cv == 1) hipLaunchKernelGGL((chunk_prep_kernel<true, 1, false, NH>), grid, block, 0, st, p);
-        else hipLaunchKernelGGL((chunk_prep_kernel<true, 2, false, NH>), grid, block, 0, st, p);
+        if (mask != nullptr) prep(std::true_type{}, std::true_type{});
+        else prep(std::true_type{}, std::false_type{});
       } else {
-        if (mask != nullptr) hipLaunchKernelGGL((chunk_prep_kernel<false, 0, true, NH>), grid, block, 0, st, p);
-        else if (cv == 0) hipLaunchKernelGGL((chunk_prep_kernel<false, 0, false, NH>), grid, block, 0, st, p);
-        else if (cv == 1) hipLaunchKernelGGL((chunk_prep_kernel<false, 1, false, NH>), grid, block, 0, st, p);
-        else hipLaunchKernelGGL((chunk_prep_kernel<false, 2, false, NH>), grid, block, 0, st, p);
+        if (mask != nullptr) prep(std::false_type{}, std::true_type{});
+        else prep(std::false_type{}, std::false_type{});
       }
     };
     // Pairs where they leave the busiest CU no more heads than single ones do
@@ -1509,10 +1526,24 @@ extern "C" int gdn_chunk_fwd_conv(const void* qkv, int64_t qkv_stride, const voi
                                   const int32_t* cu_seqlens, int64_t n_seqs, int64_t n_tok, int64_t Hk, int64_t Hv,
                                   int64_t Dk, int64_t Dv, int64_t chunk, void* workspace, size_t workspace_bytes,
                                   void* stream) {
+  return gdn_chunk_fwd_conv_masked(qkv, qkv_stride, conv_w, conv_w_dtype, conv_state_in, conv_state_out, eps, gate_mode,
+                                   gx, gy, gate_dtype, gate_stride, A_log, dt_bias, param_dtype, nullptr, state_in, y,
+                                   state_out, state_index, n_slots, cu_seqlens, n_seqs, n_tok, Hk, Hv, Dk, Dv, chunk,
+                                   workspace, workspace_bytes, stream);
+}
+
+extern "C" int gdn_chunk_fwd_conv_masked(const void* qkv, int64_t qkv_stride, const void* conv_w, int conv_w_dtype,
+                                         const void* conv_state_in, void* conv_state_out, float eps, int gate_mode,
+                                         const void* gx, const void* gy, int gate_dtype, int64_t gate_stride,
+                                         const void* A_log, const void* dt_bias, int param_dtype, const uint8_t* mask,
+                                         const float* state_in, void* y, float* state_out, const int32_t* state_index,
+                                         int64_t n_slots, const int32_t* cu_seqlens, int64_t n_seqs, int64_t n_tok,
+                                         int64_t Hk, int64_t Hv, int64_t Dk, int64_t Dv, int64_t chunk,
+                                         void* workspace, size_t workspace_bytes, void* stream) {
   const ConvArgs conv{qkv, qkv_stride, conv_w, conv_w_dtype, conv_state_in, conv_state_out, eps};
   return chunk_fwd(nullptr, nullptr, nullptr, GDN_DTYPE_BF16, gate_mode, gx, gy, gate_dtype, gate_stride, A_log,
-                   dt_bias, param_dtype, nullptr, state_in, y, state_out, state_index, n_slots, cu_seqlens, n_seqs, n_tok, Hk,
-                   Hv, Dk, Dv, chunk, workspace, workspace_bytes, stream, kPhasePrep | kPhaseScan, false, &conv);
+                   dt_bias, param_dtype, mask, state_in, y, state_out, state_index, n_slots, cu_seqlens, n_seqs, n_tok,
+                   Hk, Hv, Dk, Dv, chunk, workspace, workspace_bytes, stream, kPhasePrep | kPhaseScan, false, &conv);
 }
 
 extern "C" int gdn_chunk_fwd_noalloc(const void* q, const void* k, const void* v, int qkv_dtype, int gate_mode,

@@ -16,7 +16,7 @@ Data path per call:
                                its column slices in place
   gdn_conv_prologue            fused conv1d + SiLU + q/k norm (HIP)
   gated_delta_update           recurrent or chunked kernel (HIP); where the
-                               chunked kernel runs (long unmasked rows) the
+                               chunked kernel runs (long rows) the
                                prologue is fused into its prep instead
                                (``gdn_conv_chunked``), and for one token per
                                unmasked row of dense states into the recurrent
@@ -182,9 +182,11 @@ class GatedDeltaNet(torch.nn.Module):
 
     def _fused_prefill(self, qkv: torch.Tensor, mask) -> bool:
         """Whether a call takes the chunked kernel (``gated_delta_update``'s
-        default rule: unmasked bf16 rows of at least ``CHUNK_MIN_TOKENS``
-        tokens at 128-wide heads), with a 4-tap conv to fuse into it."""
-        return (mask is None and qkv.dtype == torch.bfloat16 and qkv.shape[1] >= CHUNK_MIN_TOKENS
+        default rule: bf16 rows of at least ``CHUNK_MIN_TOKENS`` tokens at
+        128-wide heads, masked or not), with a 4-tap conv to fuse into it
+        (masked, two rows of 300 tokens 42.7 -> 38.6 us, four of 301 51.5 ->
+        49.3, four of 512 66.1 -> 61; 17 us less on the host)."""
+        return (qkv.dtype == torch.bfloat16 and qkv.shape[1] >= CHUNK_MIN_TOKENS
                 and self.head_k_dim == 128 and self.head_v_dim == 128 and self.conv_kernel_size == 4
                 and self.conv1d_weight.dtype in (torch.bfloat16, torch.float32))
 
@@ -198,13 +200,13 @@ class GatedDeltaNet(torch.nn.Module):
         state = cache[1] if cache is not None else None
         pooled = isinstance(state, PooledBatch)
         if not verify and self._fused_prefill(qkv, mask):
-            # long unmasked rows: the conv prologue runs inside the chunked
+            # long rows: the conv prologue runs inside the chunked
             # pass's prep (bit-identical to the two launches below)
             pool = state.pool.states if pooled else state
             y, new_state, new_cs = gdn_conv_chunked(
                 qkv, self.conv1d_weight, self.num_k_heads, self.num_v_heads, self.head_k_dim, self.head_v_dim,
                 a, b, self.A_log, self.dt_bias, pool, conv_state, eps=self.rms_norm_eps,
-                state_index=state.index if pooled else None)
+                state_index=state.index if pooled else None, mask=mask)
             if cache is not None:
                 cache[0] = new_cs
                 if not pooled:

@@ -191,3 +191,32 @@ def test_mixer_prefill_takes_the_fused_path_and_matches_unfused():
         torch.cuda.synchronize()
     assert torch.equal(out1, out2)
     assert torch.equal(c1[0], c2[0]) and torch.equal(c1[1], c2[1])
+
+
+@pytest.mark.parametrize("B,S,Hk,Hv,w_dtype,kind", [
+    (4, 301, 2, 4, torch.bfloat16, "left_pad"),
+    (2, 129, 1, 3, torch.float32, "random"),
+    (1, 64, 2, 2, torch.bfloat16, "whole_row"),
+    (2, 1000, 16, 32, torch.bfloat16, "random"),  # head pairs
+    (1, 737, 16, 32, torch.float32, "left_pad"),
+])
+@pytest.mark.parametrize("with_cs", [True, False])
+def test_masked_rows_equal_unfused(B, S, Hk, Hv, w_dtype, kind, with_cs):
+    """A mask given to the fused pass and to the two launches: the same bits, and masked rows that hold NaN
+    and inf reach neither (left pads, single tokens at chunk edges and in the conv windows, a whole row)."""
+    t = _inputs(2060 + S, B, S, Hk, Hv, cs=with_cs, w_dtype=w_dtype)
+    gen = torch.Generator().manual_seed(S)
+    if kind == "left_pad":
+        pad = torch.randint(0, S, (B, 1), generator=gen)
+        mask = torch.arange(S)[None, :] >= pad
+    else:
+        mask = torch.rand(B, S, generator=gen) < (0.7 if kind == "random" else 0.0)
+    mask = mask.to(DEV)
+    t["qkv"][~mask] = float("nan")
+    t["qkv"][:, ::3][~mask[:, ::3]] = float("inf")
+    q, k, v, cs = mx.gdn_conv_prologue(t["qkv"], t["w"], Hk, Hv, D, D, t["cs"], mask)
+    y, s = mx.gated_delta_update(q, k, v, t["a"], t["b"], t["A_log"], t["dt_bias"], t["state"], mask, chunked=True)
+    got = mx.gdn_conv_chunked(t["qkv"], t["w"], Hk, Hv, D, D, t["a"], t["b"], t["A_log"], t["dt_bias"], t["state"],
+                              t["cs"], mask=mask)
+    _assert_equal(got, (y, s, cs))
+    assert torch.isfinite(got[0].float()).all() and torch.isfinite(got[1]).all()
