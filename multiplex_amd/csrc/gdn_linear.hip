@@ -297,15 +297,18 @@ linear_decode_kernel(const LinParams p) {
 // no slices meet in memory: no workspace, no ticket.
 // Reading the weights bounds it.  A is read from the L2 by every workgroup, as
 // many bytes as its weights at NB = 1 and 16 rows, so a workgroup is as wide as
-// keeps the CUs evenly busy (rows16_blocks), and the workgroups of an XCD start
-// at different chunks, so that they do not all read the same lines of A at once
-// (24576 x 4096 at 16 rows, 64 columns: 43 us without, 36 with).
+// keeps the CUs evenly busy (rows16_blocks), and neighbouring workgroups start
+// at different chunks, so that they read neither the same lines of A nor the
+// same columns of the far-apart weight rows at once (24576 x 4096 at 16 rows, 64
+// columns: 43 us without, 36 with; 4096 x 8192 at one row 14.3 us where only
+// every eighth workgroup moved on, 12.1 as here).
 // Graph-replayed at 4 rows against the sliced kernel below 64 columns and the
 // library (us; 16 rows in brackets):
 //   12352 x 2048 (NB = 4)  11.3 (11.9), 14.1 (14.4), 11.5 (11.5)
 //   10240 x 4096 (NB = 3)  15.6 (17.2), 17.7 (20.2), 18.7 (20.2)
 //    4096 x 4096 (NB = 1)   8.0  (9.8),  9.9 (10.5), 11.9 (12.3)
 //   24576 x 4096 (NB = 3)  34.1 (31.9), 35.5 (37.7), 34.4 (34.6)
+//    4096 x 8192 (NB = 1)  13.2 (17.0), 17.0,         13.6 (14.0)
 //    2048 x 4096 (NB = 1)   8.4  (9.7),  7.5  (7.8),  8.5  (8.6): half the CUs idle, so N <= 2048 is sliced
 // (84 MB in 15.6 us: 5.4 TB/s, the weights in the last-level cache).
 template <int NB>
@@ -318,7 +321,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1))) void l
   const int lr = lane & 15, lq = lane >> 4, lg8 = lq * 8;
   const int nch = p.K / KC;  // a multiple of 4 (K is one of 512): n chunks for each wave
   const int n = nch / 4;
-  const int rot = static_cast<int>(blockIdx.x / kXcds) % nch;
+  const int rot = static_cast<int>(blockIdx.x) % nch;
 
   __shared__ __align__(16) float red[4][NB][64][4];  // each wave's partial tile, lane-major
 

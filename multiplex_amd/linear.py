@@ -106,17 +106,19 @@ def linear(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     """``x @ weight.T`` (``torch.nn.functional.linear`` without a bias).
 
     Up to 16 rows of bf16, K a multiple of 512 up to 4096 and N a multiple of
-    8 above 2048, by ``gdn_linear_rows16``; the library elsewhere, and where
-    autograd, autocast or a tensor subclass needs its operator.  The line:
-    graph-replayed at 4 (16) rows, 4096 x 4096 takes 8.0 (9.8) against 11.9
-    (12.3) us, 10240 x 4096 15.6 (17.2) against 18.7 (20.2), 12352 x 2048
-    11.3 (11.9) against 11.5 (11.5); with K = 8192 or 12288 at 4096 columns
-    the library is 1 us faster, and at 2048 columns as fast.  The library
-    call itself costs the host 19 us, the launch 4.
+    8 above 2048, by ``gdn_linear_rows16``, up to 4 rows for K up to 8192 and
+    2 up to 12288; the library elsewhere, and where autograd, autocast or a
+    tensor subclass needs its operator.  The lines: graph-replayed at 4 (16)
+    rows, 4096 x 4096 takes 8.0 (9.8) against 11.9 (12.3) us, 10240 x 4096
+    15.6 (17.2) against 18.7 (20.2), 12352 x 2048 11.3 (11.9) against 11.5
+    (11.5); 4096 x 8192 at 1 / 4 / 8 rows 12.1 / 13.2 / 14.4 against 13.4 /
+    13.6 / 13.7, 4096 x 12288 at 1 / 2 / 4 rows 16.6 / 17.3 / 18.5 against
+    17.5 / 17.7 / 17.7; at 2048 columns the library is as fast.  The library call
+    itself costs the host 19 us, the launch 4.
     """
     N, K = weight.shape
     rows = x.numel() // K if K else 0
-    if (1 <= rows <= 16 and 512 <= K <= 4096 and K % 512 == 0 and N > 2048 and N % 8 == 0
+    if (1 <= rows <= (16 if K <= 4096 else 4 if K <= 8192 else 2) and 512 <= K <= 12288 and K % 512 == 0 and N > 2048 and N % 8 == 0
             and x.dtype is torch.bfloat16 and weight.dtype is torch.bfloat16 and x.is_cuda and weight.is_cuda
             and x.shape[-1] == K and x.is_contiguous() and weight.is_contiguous()
             and type(x) is torch.Tensor and type(weight) in (torch.Tensor, torch.nn.Parameter)

@@ -49,7 +49,8 @@ def test_linear_decode_matches_float64(M, N, K):
 
 
 @pytest.mark.parametrize("M,N,K", [(1, 2056, 512), (16, 4096, 4096), (5, 4104, 1536), (16, 8200, 512),
-                                   (7, 10240, 4096), (3, 12352, 2048), (16, 24584, 1024)])
+                                   (7, 10240, 4096), (3, 12352, 2048), (16, 24584, 1024), (4, 4096, 8192),
+                                   (2, 4096, 12288)])
 def test_linear_up_to_16_rows_matches_float64(M, N, K):
     """One workgroup per tile of 16 to 64 columns: tiles with a ragged last one,
     one to eight chunks of K a wave.  fp32 sums in another order, as above."""
