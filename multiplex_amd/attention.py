@@ -36,7 +36,7 @@ from typing import List, Optional, Sequence
 import torch
 
 from . import _lib
-from .gated_delta import _dtype_code, _ptr, _require_device, _stream
+from .gated_delta import _dtype_code, _on_device, _ptr, _require_device, _stream
 from .linear import linear
 
 __all__ = [
@@ -343,7 +343,8 @@ class KVCache:
         p = self.pos0
         if not p.is_cuda or p.dtype is not torch.int32 or not p.is_contiguous() or not -2**31 <= delta < 2**31:
             return False
-        _lib.call("gdn_pos_add", p.data_ptr(), p.numel(), delta, lo, _stream(p.device))
+        with _on_device(p.device):
+            _lib.call("gdn_pos_add", p.data_ptr(), p.numel(), delta, lo, _stream(p.device))
         return True
 
     def filter(self, keep: Sequence[int]) -> None:
