@@ -32,7 +32,7 @@ from typing import Optional
 import torch
 
 from . import _lib
-from .gated_delta import _dtype_code, _ptr, _require_device, _stream
+from .gated_delta import _dtype_code, _on_device, _ptr, _require_device, _stream
 
 __all__ = ["linear", "DECODE_MAX_ROWS", "FUSED_NORM_MAX_ROWS", "DecodeWorkspace", "linear_decode",
            "gated_norm_linear_decode", "linear_decode_workspace_bytes", "decode_shape_ok"]
@@ -126,10 +126,17 @@ def linear(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
             and not (torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad))):
         xp, wp = x.data_ptr(), weight.data_ptr()
         if xp % 16 == 0 and wp % 16 == 0:
-            out = torch.empty(*x.shape[:-1], N, dtype=torch.bfloat16, device=x.device)
-            _lib.call("gdn_linear_rows16", xp, K, wp, out.data_ptr(), N, rows, N, K, _stream(x.device))
-            return out
+            return _rows16(x, weight, rows)
     return torch.nn.functional.linear(x, weight)
+
+
+def _rows16(x, weight, rows):
+    N, K = weight.shape
+    dev = x.device
+    out = torch.empty(*x.shape[:-1], N, dtype=torch.bfloat16, device=dev)
+    with _on_device(dev):
+        _lib.call("gdn_linear_rows16", x.data_ptr(), K, weight.data_ptr(), out.data_ptr(), N, rows, N, K, _stream(dev))
+    return out
 
 
 def linear_decode(x: torch.Tensor, weight: torch.Tensor, *, out: Optional[torch.Tensor] = None,

@@ -13,7 +13,7 @@ import pytest
 import torch
 
 import multiplex_amd as mx
-from multiplex_amd import _lib, attention, gated_delta
+from multiplex_amd import _lib, attention, gated_delta, linear
 
 
 @pytest.fixture
@@ -32,7 +32,7 @@ def launches(monkeypatch):
         made.append(name)
 
     monkeypatch.setattr(_lib, "call", call)
-    for mod in (attention,):
+    for mod in (attention, linear):
         monkeypatch.setattr(mod, "_on_device", enter, raising=False)
         monkeypatch.setattr(mod, "_stream", lambda dev: 0)
         monkeypatch.setattr(mod, "_require_device", lambda tensors, names: torch.device("cpu"))
@@ -67,3 +67,9 @@ def test_cache_offsets(launches):
     c.advance(5)
     c.trim(2)
     assert c.lengths == [3, 3, 3] and launches == ["gdn_pos_add"] * 2
+
+
+def test_projection_of_few_rows(launches):
+    x, w = torch.zeros(3, 1, 512, dtype=torch.bfloat16), torch.zeros(2056, 512, dtype=torch.bfloat16)
+    assert linear._rows16(x, w, 3).shape == (3, 1, 2056)
+    assert launches == ["gdn_linear_rows16"]
