@@ -40,6 +40,7 @@ __all__ = ["linear", "DECODE_MAX_ROWS", "FUSED_NORM_MAX_ROWS", "DecodeWorkspace"
 DECODE_MAX_ROWS = 64
 FUSED_NORM_MAX_ROWS = 16  # where the fused norm + projection beats the norm kernel plus the library GEMM
 _K_SLICE = 512
+_MAX_COLUMNS = 262144  # gdn_linear_rows16's limit
 
 
 def linear_decode_workspace_bytes(M: int, N: int, K: int) -> int:
@@ -118,8 +119,7 @@ def linear(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     """
     N, K = weight.shape
     rows = x.numel() // K if K else 0
-    if (1 <= rows <= (16 if K <= 4096 else 4 if K <= 8192 else 2) and 512 <= K <= 12288 and K % 512 == 0 and N > 2048 and N % 8 == 0
-            and x.dtype is torch.bfloat16 and weight.dtype is torch.bfloat16 and x.is_cuda and weight.is_cuda
+    if (_rows16_shape(rows, N, K) and x.dtype is torch.bfloat16 and weight.dtype is torch.bfloat16 and x.is_cuda and weight.is_cuda
             and x.shape[-1] == K and x.is_contiguous() and weight.is_contiguous()
             and type(x) is torch.Tensor and type(weight) in (torch.Tensor, torch.nn.Parameter)
             and x.device == weight.device and not torch.is_autocast_enabled()
@@ -128,6 +128,13 @@ def linear(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
         if xp % 16 == 0 and wp % 16 == 0:
             return _rows16(x, weight, rows)
     return torch.nn.functional.linear(x, weight)
+
+
+def _rows16_shape(rows, N, K) -> bool:
+    """The sizes :func:`linear` gives to ``gdn_linear_rows16`` (which refuses
+    more than ``_MAX_COLUMNS`` columns)."""
+    return (1 <= rows <= (16 if K <= 4096 else 4 if K <= 8192 else 2) and 512 <= K <= 12288 and K % _K_SLICE == 0
+            and 2048 < N <= _MAX_COLUMNS and N % 8 == 0)
 
 
 def _rows16(x, weight, rows):

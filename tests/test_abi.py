@@ -11,7 +11,7 @@ from pathlib import Path
 import pytest
 import torch
 
-from multiplex_amd import _lib
+from multiplex_amd import _lib, linear
 
 ROOT = Path(__file__).resolve().parents[1]
 HEADER = ROOT / "include" / "gdn.h"
@@ -257,3 +257,10 @@ def test_attention_entry_points_reject_bad_arguments(lib):
     assert lib.gdn_rms_norm(FAKE, None, None, None, _lib.DTYPE_F32, FAKE, 0, 4, 16, 1e-6, None) == _lib.ERR_INVALID
     assert lib.gdn_silu_mul(FAKE, FAKE, 4, 12, None) == _lib.ERR_INVALID
     assert lib.gdn_silu_mul(FAKE, FAKE, 0, 16, None) == _lib.OK
+
+
+@pytest.mark.parametrize("N", [2056, 262136, 262144, 262152, 1 << 20])
+def test_few_row_projections_stop_at_the_column_limit(lib, N):
+    """linear() gives the library call what gdn_linear_rows16 refuses."""
+    taken = lib.gdn_linear_rows16(FAKE, 2048, None, FAKE, N, 4, N, 2048, None) != _lib.ERR_UNSUPPORTED
+    assert linear._rows16_shape(4, N, 2048) == taken == (N <= 262144)
