@@ -30,6 +30,7 @@ from __future__ import annotations
 from typing import Optional
 
 import torch
+import torch.autograd.forward_ad as forward_ad
 
 from . import _lib
 from .gated_delta import _dtype_code, _on_device, _ptr, _require_device, _stream
@@ -108,8 +109,8 @@ def linear(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
 
     Up to 16 rows of bf16, K a multiple of 512 up to 4096 and N a multiple of
     8 above 2048, by ``gdn_linear_rows16``, up to 4 rows for K up to 8192 and
-    2 up to 12288; the library elsewhere, and where autograd, autocast or a
-    tensor subclass needs its operator.  The lines: graph-replayed at 4 (16)
+    2 up to 12288; the library elsewhere, and where differentiation, autocast, a
+    function transform or a tensor subclass needs its operator.  The lines: graph-replayed at 4 (16)
     rows, 4096 x 4096 takes 8.0 (9.8) against 11.9 (12.3) us, 10240 x 4096
     15.6 (17.2) against 18.7 (20.2), 12352 x 2048 11.3 (11.9) against 11.5
     (11.5); 4096 x 8192 at 1 / 4 / 8 rows 12.1 / 13.2 / 14.4 against 13.4 /
@@ -119,15 +120,31 @@ def linear(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     """
     N, K = weight.shape
     rows = x.numel() // K if K else 0
-    if (_rows16_shape(rows, N, K) and x.dtype is torch.bfloat16 and weight.dtype is torch.bfloat16 and x.is_cuda and weight.is_cuda
-            and x.shape[-1] == K and x.is_contiguous() and weight.is_contiguous()
-            and type(x) is torch.Tensor and type(weight) in (torch.Tensor, torch.nn.Parameter)
-            and x.device == weight.device and not torch.is_autocast_enabled()
-            and not (torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad))):
+    if (_rows16_shape(rows, N, K) and x.dtype is torch.bfloat16 and weight.dtype is torch.bfloat16
+            and x.is_cuda and weight.is_cuda and x.shape[-1] == K and not _needs_operator(x, weight)
+            and x.is_contiguous() and weight.is_contiguous() and x.device == weight.device):
         xp, wp = x.data_ptr(), weight.data_ptr()
         if xp % 16 == 0 and wp % 16 == 0:
             return _rows16(x, weight, rows)
     return torch.nn.functional.linear(x, weight)
+
+
+_transform_level = getattr(torch._C._functorch, "maybe_current_level", None)
+
+
+def _needs_operator(x, weight) -> bool:
+    """Whether something follows or replaces the operator on these operands: a
+    recorded gradient, a forward-mode tangent (its tensors are plain ones that
+    ask for no gradient), a function transform (vmap, jvp, grad), autocast, a
+    tensor subclass."""
+    if (type(x) is not torch.Tensor or type(weight) not in (torch.Tensor, torch.nn.Parameter)
+            or torch.is_autocast_enabled() or (torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad))):
+        return True
+    if _transform_level is None or _transform_level() is not None:
+        return True
+    # (outside a dual level, -1, no tensor has a tangent)
+    return getattr(forward_ad, "_current_level", 0) >= 0 and any(
+        forward_ad.unpack_dual(t).tangent is not None for t in (x, weight))
 
 
 def _rows16_shape(rows, N, K) -> bool:

@@ -19,6 +19,7 @@ from __future__ import annotations
 import numpy as np
 import pytest
 import torch
+import torch.autograd.forward_ad as fwad
 
 import multiplex_amd as mx
 from multiplex_amd import linear as lin
@@ -77,6 +78,19 @@ def test_linear_leaves_other_calls_to_the_library():
     x = _bf16(gen, 4, 1024).to(DEV).requires_grad_()
     lin.linear(x, W).sum().backward()
     assert x.grad is not None
+
+
+def test_linear_keeps_forward_mode_tangents():
+    """Forward-mode operands are plain tensors without requires_grad."""
+    gen = torch.Generator().manual_seed(96)
+    x, W = _bf16(gen, 4, 1024).to(DEV), _bf16(gen, 4096, 1024, scale=1 / 32).to(DEV)
+    dx, dW = _bf16(gen, 4, 1024).to(DEV), _bf16(gen, 4096, 1024, scale=1 / 32).to(DEV)
+    fl = torch.nn.functional.linear
+    with torch.no_grad(), fwad.dual_level():
+        for a, b in ((fwad.make_dual(x, dx), W), (x, fwad.make_dual(W, dW))):
+            got, want = fwad.unpack_dual(lin.linear(a, b)), fwad.unpack_dual(fl(a, b))
+            assert torch.equal(got.primal, want.primal) and torch.equal(got.tangent, want.tangent)
+        assert fwad.unpack_dual(lin.linear(x, W)).tangent is None
 
 
 def test_linear_decode_reads_column_slices_and_writes_strided_rows():
