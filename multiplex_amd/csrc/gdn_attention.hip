@@ -868,7 +868,7 @@ __global__ __launch_bounds__(256 * KG) void attn_prefill_kernel(const AttnParams
     const int r = row0 + 32 * rg + 16 * rt + lr;
     if (r >= n_rows) return;
     if (p.n_split == 1) {
-      const float inv_l = lt[rt] > 0.0f ? 1.0f / lt[rt] : 0.0f;
+      const float inv_l = 1.0f / lt[rt];  // (l = 0: every score is -inf, whose softmax is NaN)
 #pragma unroll
       for (int j = 0; j < NJ; ++j) store_out4<D>(p, b, r / g, hkv * g + r % g, 16 * j + 4 * lq, o[rt][j], inv_l);
       return;
@@ -974,7 +974,8 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(const AttnParams p) {
       }
     }
   }
-  const float inv_l = lsum > 0.0f ? 1.0f / lsum : 0.0f;
+  // l = 0: every score is -inf, whose softmax is NaN (zeros in the kernel of fewer rows)
+  const float inv_l = n_rows >= kPrefillRows || lsum > 0.0f ? 1.0f / lsum : 0.0f;
   const int t = r / g, hq = hkv * g + r % g;
   if constexpr (EPL == 4) {
     store_out4<D>(p, b, t, hq, EPL * lane, acc, inv_l);

@@ -208,6 +208,23 @@ def test_attention_matches_oracle(name):
     assert _row_errs(got, ref).max() < ATT_TOL
 
 
+@pytest.mark.parametrize("T,n_split,heads", [(130, 1, (16, 4, 256)), (130, 2, (16, 4, 256)), (300, 1, (16, 4, 128))])
+def test_long_prefill_of_a_row_whose_scores_are_all_minus_infinity(T, n_split, heads):
+    """The softmax of no finite score is NaN, as the oracle's; rows that see other keys too are not touched."""
+    Hq, Hkv, D = heads
+    gen = torch.Generator().manual_seed(84)
+    kc, vc, q = _bf16(gen, 1, Hkv, T, D), _bf16(gen, 1, Hkv, T, D), _bf16(gen, 1, T, Hq, D)
+    q[..., 0] = q[..., 0].abs() + 0.5
+    kc[:, :, 0, 0] = float("-inf")  # key 0, the only one that token 0 sees
+    out = att.attn_fwd(q.to(DEV), kc.to(DEV), vc.to(DEV), torch.zeros(1, dtype=torch.int32, device=DEV), T,
+                       n_split=n_split)
+    with np.errstate(invalid="ignore"):
+        ref = oa.attention(_np(q), _np(kc), _np(vc), [0], D ** -0.5)
+    got = _np(out)
+    assert np.isnan(ref[:, 0]).all() and np.isnan(got[:, 0]).all()
+    assert _row_errs(got[:, 1:], ref[:, 1:]).max() < ATT_TOL
+
+
 @pytest.mark.parametrize("B", [1, 256, 257])
 def test_cache_offsets_advance_and_roll_back(B):
     """Exact: the device offsets follow the host lengths, and a rollback stops
