@@ -439,18 +439,23 @@ class Attention(torch.nn.Module):
         self.k_norm.weight.copy_(k_norm)
 
     def _splits(self, B: int, T: int, L: int) -> int:
-        """Key ranges per row, where the rows alone leave CUs idle (measured
-        at 4 kv-heads of 256, us with one range and with the rule's).
+        """Key ranges per row, where the rows alone leave CUs idle (graph-
+        replayed at 4 kv-heads of 256, us with one range and with the rule's).
 
         At least 512 rows (tokens x heads of a group) a kv-head: the 128-row
         tiles' workgroups, one per CU, times the ranges fit the CUs, each at
-        least 256 keys of the prefix (512 tokens over 4096: 129 -> 61; 128
-        over 8192: 216 -> 43; 1024 over none stays whole: 42, two ranges 47).
-        Up to 16 rows (decode, draft verify): about one workgroup per CU, more
-        than 64 keys (one token over 1024: 36 -> 14, over 256: 13.1 -> 11.6,
-        over 128: 9.9, two ranges 11.0).  Between: 64-row tiles, two workgroups per CU; at least
-        128 keys up to one workgroup per CU and 256 beyond (8 tokens over
-        16384: 853 -> 35; 32 over 1024: 60 -> 20; 64 over 8192: 430 -> 45).
+        least 256 keys of the prefix (512 tokens over 4096: 122 -> 55; 128
+        over 8192: 212 -> 39; 1024 over none stays whole: 38, two ranges 43).
+        Up to 16 rows (decode, draft verify): at most about one workgroup per
+        CU, 128 or more keys (one token over 1024: 30.3 -> 11.4; of four over
+        4001: 120 -> 19.6).  Between: 64-row tiles, two workgroups per CU; at
+        least 128 keys up to one workgroup per CU and 256 beyond (8 tokens
+        over 16384: 828 -> 31; 32 over 1024: 53 -> 16; 64 over 8192: 417 -> 40).
+
+        A range is whole blocks of 64 keys (the launch rounds its length up),
+        and there are only as many ranges as hold keys: ranges without any
+        were launched all the same (one token over 4001: 61 ranges for 32
+        with keys, 15.4 -> 13.5).
         """
         if self.n_split is not None:
             return self.n_split
@@ -459,11 +464,15 @@ class Attention(torch.nn.Module):
         rows = T * (self.Hq // self.Hkv)
         if rows >= 512:
             n = B * self.Hkv * -(-rows // 128)
-            return max(1, min(self._cus // n, (L - T) // 256))
-        if rows <= 16:
-            return max(1, min(round(self._cus / (B * self.Hkv)), L // 64 - 1))
-        n = B * self.Hkv * -(-rows // 64)
-        return max(1, min(self._cus // n, L // 128), min(2 * self._cus // n, L // 256))
+            ranges = max(1, min(self._cus // n, (L - T) // 256))
+        elif rows <= 16:
+            ranges = max(1, min(round(self._cus / (B * self.Hkv)), L // 64 - 1))
+        else:
+            n = B * self.Hkv * -(-rows // 64)
+            ranges = max(1, min(self._cus // n, L // 128), min(2 * self._cus // n, L // 256))
+        blocks = -(-L // 64)
+        of_range = max(1, -(-(-(-L // ranges)) // 64))  # as gdn_attn_fwd takes it
+        return max(1, -(-blocks // of_range))
 
     def forward(self, x: torch.Tensor, cache: KVCache) -> torch.Tensor:
         B, T, _ = x.shape

@@ -259,6 +259,19 @@ def test_split_keys_agree_with_one_range():
     assert _row_errs(_np(b), _np(a)).max() < 4e-3
 
 
+@pytest.mark.parametrize("T,L,n", [(1, 1024, 15), (4, 4001, 61), (16, 4112, 60), (128, 8320, 16)])
+def test_ranges_without_keys_do_not_change_the_result(T, L, n):
+    """Ranges are whole 64-key blocks, so n of them may leave the last ones without keys: fewer ranges of
+    the same length are the same sums, bit for bit."""
+    gen = torch.Generator().manual_seed(85)
+    q, kc, vc = (_bf16(gen, 1, *s).to(DEV) for s in ((T, 16, 256), (4, L, 256), (4, L, 256)))
+    pos0 = torch.full((1,), L - T, dtype=torch.int32, device=DEV)
+    keys = -(-(-(-L // n)) // 64) * 64
+    fewer = -(-L // keys)
+    assert fewer < n and -(-(-(-L // fewer)) // 64) * 64 == keys
+    assert torch.equal(att.attn_fwd(q, kc, vc, pos0, L, n_split=n), att.attn_fwd(q, kc, vc, pos0, L, n_split=fewer))
+
+
 ARGS = mx.AttentionArgs(hidden_size=512, num_attention_heads=8, num_key_value_heads=2, head_dim=256,
                         intermediate_size=768, rms_norm_eps=1e-6, partial_rotary_factor=0.25, rope_theta=1.0e7)
 
