@@ -302,15 +302,18 @@ linear_decode_kernel(const LinParams p) {
 // same columns of the far-apart weight rows at once (24576 x 4096 at 16 rows, 64
 // columns: 43 us without, 36 with; 4096 x 8192 at one row 14.3 us where only
 // every eighth workgroup moved on, 12.1 as here).
-// Graph-replayed at 4 rows against the sliced kernel below 64 columns and the
-// library (us; 16 rows in brackets):
-//   12352 x 2048 (NB = 4)  11.3 (11.9), 14.1 (14.4), 11.5 (11.5)
-//   10240 x 4096 (NB = 3)  15.6 (17.2), 17.7 (20.2), 18.7 (20.2)
-//    4096 x 4096 (NB = 1)   8.0  (9.8),  9.9 (10.5), 11.9 (12.3)
-//   24576 x 4096 (NB = 3)  34.1 (31.9), 35.5 (37.7), 34.4 (34.6)
-//    4096 x 8192 (NB = 1)  13.2 (17.0), 17.0,         13.6 (14.0)
-//    2048 x 4096 (NB = 1)   8.4  (9.7),  7.5  (7.8),  8.5  (8.6): half the CUs idle, so N <= 2048 is sliced
-// (84 MB in 15.6 us: 5.4 TB/s, the weights in the last-level cache).
+// Graph-replayed at 4 rows (16 in brackets) against the sliced kernel below and
+// the library, the weights read from memory (us; linear.py has more sizes, and
+// the times with one weight that stays in the last-level cache):
+//   12352 x 2048 (NB = 4)  11.1 (12.2), 15.0 (16.3), 15.1 (15.1)
+//   10240 x 4096 (NB = 3)  16.1 (18.4), 21.4 (23.9), 24.8 (25.0)
+//    4096 x 4096 (NB = 1)   8.0  (9.9), 11.5 (12.1), 14.7 (14.7)
+//   24576 x 4096 (NB = 3)  34.1 (36.5), 45.2 (46.9), 42.8 (43.1)
+//    4096 x 8192 (NB = 1)  15.5 (17.4), 17.6 (21.0), 15.5 (16.0)
+//    4096 x 12288 (NB = 1) 18.7 (24.9), 25.3 (29.2), 21.1 (21.4)
+//    2048 x 4096 (NB = 1)   7.7  (9.6),  8.9  (9.3), 14.9 (14.8): half the CUs idle; from the cache 7.2 (9.0),
+//                           6.9 (7.3), 8.0 (8.1), so N <= 2048 is sliced
+// (84 MB in 16.1 us: 5.2 TB/s from memory, 15.1 us from the cache.)
 template <int NB>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1))) void linear_rows16_kernel(const LinParams p) {
   constexpr int KC = 128, SQ = KC / 32;  // columns of K per chunk, k-steps

@@ -107,16 +107,10 @@ def _launch(x, gate, norm_weight, eps, head_dim, weight, out, workspace):
 def linear(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     """``x @ weight.T`` (``torch.nn.functional.linear`` without a bias).
 
-    Up to 16 rows of bf16, K a multiple of 512 up to 4096 and N a multiple of
-    8 above 2048, by ``gdn_linear_rows16``, up to 4 rows for K up to 8192 and
-    2 up to 12288; the library elsewhere, and where differentiation, autocast, a
-    function transform or a tensor subclass needs its operator.  The lines: graph-replayed at 4 (16)
-    rows, 4096 x 4096 takes 8.0 (9.8) against 11.9 (12.3) us, 10240 x 4096
-    15.6 (17.2) against 18.7 (20.2), 12352 x 2048 11.3 (11.9) against 11.5
-    (11.5); 4096 x 8192 at 1 / 4 / 8 rows 12.1 / 13.2 / 14.4 against 13.4 /
-    13.6 / 13.7, 4096 x 12288 at 1 / 2 / 4 rows 16.6 / 17.3 / 18.5 against
-    17.5 / 17.7 / 17.7; at 2048 columns the library is as fast.  The library call
-    itself costs the host 19 us, the launch 4.
+    A few rows of bf16 (:func:`_rows16_shape` has the sizes) by
+    ``gdn_linear_rows16``; the library elsewhere, and where differentiation,
+    autocast, a function transform or a tensor subclass needs its operator.
+    The call costs the host 6.7 us, the library's 17.6.
     """
     N, K = weight.shape
     rows = x.numel() // K if K else 0
@@ -149,9 +143,30 @@ def _needs_operator(x, weight) -> bool:
 
 def _rows16_shape(rows, N, K) -> bool:
     """The sizes :func:`linear` gives to ``gdn_linear_rows16`` (which refuses
-    more than ``_MAX_COLUMNS`` columns)."""
-    return (1 <= rows <= (16 if K <= 4096 else 4 if K <= 8192 else 2) and 512 <= K <= 12288 and K % _K_SLICE == 0
-            and 2048 < N <= _MAX_COLUMNS and N % 8 == 0)
+    more than ``_MAX_COLUMNS`` columns).
+
+    The lines follow graph-replayed times with the weights read from memory,
+    as those of a model's layers are (each call another of 600 MB of them);
+    behind them, after the slash, calls of one weight that stays in the
+    last-level cache, where the library gains more.  us, against the library's:
+      K to 4096, 16 rows:  4096 x 4096 9.9 / 9.3, 14.7 / 11.6 (4 rows 8.0 / 7.3, 14.7 / 11.3);
+        10240 x 4096 18.4 / 16.8, 25.0 / 19.6; 12352 x 2048 12.2 / 11.5, 15.1 / 10.8 (8 rows 11.4 / 10.7,
+        15.1 / 10.8); 6144 x 4096 13.6 / 12.9, 14.4 / 11.3.  Of 120 sizes from 512 to 4096 by 2056 to 24576
+        it is the slower one at 13, by 10% at most (K = 2560 and 3584 at 4608 to 8192 columns, 16384 columns);
+        with the weight in the cache at 75, by 57% at most (K = 2560 at 4608 to 6144 columns)
+      K to 8192, 4 rows:   4096 x 8192 15.5 / 12.4, 15.5 / 13.0; 12288 x 8192 35.3 / 29.6, 39.5 / 31.4
+      K to 12288, 2 rows:  4096 x 12288 18.4 / 16.2, 21.0 / 17.0; 16384 x 12288 69.9 / 69.1, 82.4 / 86.4
+      K over 4096 at 4104 to 8192 columns, whose tiles load the CUs unevenly or (8192 wide) are read
+        7168 to 16384 bytes apart, is the library's: 5120 x 5120 at 4 rows 14.5 / 13.0, 14.0 / 11.5;
+        6144 x 8192 23.2 / 19.3, 21.4 / 17.9; 8192 x 8192 32.0 / 20.3, 28.9 / 21.7
+    """
+    if K <= 4096:
+        most = 16
+    elif 4096 < N <= 8192:
+        most = 0
+    else:
+        most = 4 if K <= 8192 else 2
+    return 1 <= rows <= most and 512 <= K <= 12288 and K % _K_SLICE == 0 and 2048 < N <= _MAX_COLUMNS and N % 8 == 0
 
 
 def _rows16(x, weight, rows):

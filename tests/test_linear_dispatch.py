@@ -48,3 +48,16 @@ def test_function_transforms_need_the_operator(transform):
     else:
         torch.func.vmap(f)(w[None])
     assert seen == [True]
+
+
+@pytest.mark.parametrize("rows,N,K,taken", [
+    (16, 2056, 512, True), (16, 24576, 4096, True), (17, 4096, 4096, False), (0, 4096, 4096, False),
+    (1, 2048, 4096, False), (1, 4100, 4096, False), (1, 4096, 4097, False), (1, 4096, 256, False),
+    (4, 4096, 8192, True), (5, 4096, 8192, False), (2, 4096, 12288, True), (3, 4096, 12288, False),
+    (1, 4096, 12800, False), (2, 8200, 12288, True), (4, 12288, 4608, True),
+    # over 4096 wide, more than one 16-column tile a CU and at most two
+    (1, 4104, 4608, False), (4, 5120, 5120, False), (1, 6144, 8192, False), (2, 8192, 8192, False),
+    (2, 8192, 12288, False), (16, 8192, 4096, True),
+])
+def test_sizes_given_to_the_kernel(rows, N, K, taken):
+    assert linear._rows16_shape(rows, N, K) is taken
