@@ -408,6 +408,14 @@ class RMSNorm(torch.nn.Module):
         return rms_norm(x, self.weight, self.eps, residual=residual, out=out)
 
 
+# Rows of a workgroup's tile -> (us a 64-key block of its chain takes, us a MB
+# of partial results costs) at head dims up to 128 and 256; the merge costs
+# another 3.5.  Fitted to graph-replayed times of 4264 sizes (7 head layouts, 1
+# to 48 rows, 1 to 1024 tokens, up to 9000 keys) with one range and with several:
+# the choice is the slower one at 39 of them, by 2 to 11%.
+_SPLIT_US = {16: ((1.07, 0.9), (1.85, 1.1)), 64: ((1.83, 0.9), (3.25, 0.7)), 128: ((1.1, 0.8), (1.5, 0.45))}
+
+
 class Attention(torch.nn.Module):
     """Qwen3.5 gated full attention (mlx-lm ``qwen3_5`` Attention).
 
@@ -446,11 +454,16 @@ class Attention(torch.nn.Module):
         tiles' workgroups, one per CU, times the ranges fit the CUs, each at
         least 256 keys of the prefix (512 tokens over 4096: 122 -> 55; 128
         over 8192: 212 -> 39; 1024 over none stays whole: 38, two ranges 43).
-        Up to 16 rows (decode, draft verify): at most about one workgroup per
-        CU, 128 or more keys (one token over 1024: 30.3 -> 11.4; of four over
-        4001: 120 -> 19.6).  Between: 64-row tiles, two workgroups per CU; at
+        Up to 16 rows (decode, draft verify): one workgroup per CU, 128 or
+        more keys (one token over 1024: 30.3 -> 11.4; of four over 4001:
+        120 -> 19.6), or about one of 512 or more.  Between: 64-row tiles, two workgroups per CU; at
         least 128 keys up to one workgroup per CU and 256 beyond (8 tokens
         over 16384: 828 -> 31; 32 over 1024: 53 -> 16; 64 over 8192: 417 -> 40).
+
+        The blocks that a workgroup's chain is then shorter by have to pay
+        for the partial results, which are written, read and merged
+        (:data:`_SPLIT_US`).  Where they do not, one range: 256 tokens of four
+        rows over 512 at heads of 128, 21 us, two ranges 34.
 
         A range is whole blocks of 64 keys (the launch rounds its length up),
         and there are only as many ranges as hold keys: ranges without any
@@ -464,15 +477,22 @@ class Attention(torch.nn.Module):
         rows = T * (self.Hq // self.Hkv)
         if rows >= 512:
             n = B * self.Hkv * -(-rows // 128)
+            tile = 128
             ranges = max(1, min(self._cus // n, (L - T) // 256))
         elif rows <= 16:
-            ranges = max(1, min(round(self._cus / (B * self.Hkv)), L // 64 - 1))
+            tile = 16
+            n = B * self.Hkv
+            ranges = max(1, min(round(self._cus / n), max(self._cus // n, L // 512), L // 64 - 1))
         else:
             n = B * self.Hkv * -(-rows // 64)
+            tile = 64
             ranges = max(1, min(self._cus // n, L // 128), min(2 * self._cus // n, L // 256))
         blocks = -(-L // 64)
         of_range = max(1, -(-(-(-L // ranges)) // 64))  # as gdn_attn_fwd takes it
-        return max(1, -(-blocks // of_range))
+        ranges = max(1, -(-blocks // of_range))
+        block_us, mb_us = _SPLIT_US[tile][self.D > 128]
+        partials = 4e-6 * B * self.Hkv * rows * ranges * self.D  # MB
+        return ranges if block_us * (blocks - of_range) > 3.5 + mb_us * partials else 1
 
     def forward(self, x: torch.Tensor, cache: KVCache) -> torch.Tensor:
         B, T, _ = x.shape
