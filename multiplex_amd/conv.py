@@ -247,7 +247,9 @@ def gdn_conv_chunked(qkv: torch.Tensor, conv_weight: torch.Tensor, num_k_heads: 
     return outs
 
 
-CONV_DECODE_MAX_ROWS = 64  # where one launch is no slower than two (conv_decode_kernel's figures)
+# Where one launch is no slower than two: rows, and rows x v-heads (conv_decode_kernel's figures).
+CONV_DECODE_MAX_ROWS = 64
+CONV_DECODE_MAX_HEADS = 2048
 
 
 def gdn_conv_decode(qkv, conv_weight, num_k_heads, num_v_heads, head_k_dim, head_v_dim, a, b, A_log, dt_bias, state,
@@ -257,14 +259,14 @@ def gdn_conv_decode(qkv, conv_weight, num_k_heads, num_v_heads, head_k_dim, head
     ``gated_delta_update``, bit for bit.  Arguments as there; dense states.
 
     Returns ``(y, new_state, new_conv_state)``, or None for operands it does
-    not take (other types, head sizes, taps or layouts, more than 64 rows):
+    not take (other types, head sizes, taps or layouts, more rows or heads):
     the caller then runs the two, which check them.
     """
     B, S, C = qkv.shape
     Hk, Hv, D = num_k_heads, num_v_heads, 128
     bf16 = torch.bfloat16
-    if (S != 1 or not 1 <= B <= CONV_DECODE_MAX_ROWS or head_k_dim != D or head_v_dim != D
-            or C != 2 * Hk * D + Hv * D or Hv % Hk != 0 or Hv > 65535
+    if (S != 1 or not 1 <= B <= CONV_DECODE_MAX_ROWS or B * Hv > CONV_DECODE_MAX_HEADS or head_k_dim != D or head_v_dim != D
+            or C != 2 * Hk * D + Hv * D or Hv % Hk != 0
             or qkv.dtype is not bf16 or a.dtype is not bf16 or b.dtype is not bf16
             or conv_weight.dtype is not bf16 or conv_weight.shape != (C, 4) or not conv_weight.is_contiguous()
             or a.shape != (B, 1, Hv) or b.shape != (B, 1, Hv) or A_log.shape != (Hv,) or dt_bias.shape != (Hv,)

@@ -369,7 +369,8 @@ __global__ __launch_bounds__(256) void recurrent_kernel(const RecParams p) {
 // with q, k and v through memory between them.  Graph-replayed at Hv = 32, the
 // two launches against U = 2 / 4 / 8 (us): 1 row 5.6, 3.8 / 4.1 / 4.6; 4 rows
 // 7.3, 5.4 / 5.1 / 5.4; 8 rows 10.0, 8.0 / 7.9 / 6.9 (4.9 TB/s); 16 rows 15.1,
-// 14.6 / 14.0 / 12.9; 64 rows 47.8, 50.6 / 48.1 / 47.5.
+// 14.6 / 14.0 / 12.9; 64 rows 47.8, 50.6 / 48.1 / 47.5.  Beyond 2048 heads the two
+// launches win (Hv = 64: 32 rows 47.4, 47.7; 48 rows 69.0, 70.4; 64 rows 90.0, 93.2).
 struct ConvDecodeParams {
   const uint16_t* qkv;  // [B] rows of C = 2 Hk 128 + Hv 128 channels, ld apart
   int64_t ld;
