@@ -95,11 +95,15 @@ struct RowVec {
 // lane only, so exp2 and sincos -- most of the arithmetic, computed per head
 // it bounded the kernel at 70.6 us for 4096 tokens of 16 + 2 x 4 heads --
 // run once for the NH heads, whose rows are all loaded before the first is
-// used and whose chains overlap.  A wave with more heads runs longer, so few
-// tokens take few heads a wave (graph-replayed, us, NH = 1 / 3 / 6):
-//   1 token 5.7 / 6.8 / 7.9, 128 tokens 6.9 / 7.2 / 8.3, 256 8.7 / 7.8 / 8.6,
-//   512 12.4 / 9.8 / 9.6, 1024 19.5 / 13.5 / 12.6, 4096 59.1 / 33.2 / 28.3
-// (100 MB: 3.6 TB/s).
+// used and whose chains overlap.  A wave with more heads runs longer, so calls
+// of few rows (tokens x heads) take few heads a wave (graph-replayed, us, NH =
+// 1 / 3 / 6; a wave per head with the angles of its own before them):
+//   16 + 2 x 4 heads of 256:   1 token 3.3, 3.5 / 4.3 / 5.5;  160 tokens (3840 rows) 5.4, 5.0 / 5.2 / 5.9;
+//      200 (4800) 5.9, 5.5 / 5.3 / 6.0;  600 (14400) 12.3, 11.0 / 7.9 / 8.0;  700 (16800) 13.7, 12.3 / 8.8 / 8.2;
+//      2048 34.1, 29.1 / 17.1 / 16.2
+//   4 + 2 x 1 of 256:        600 tokens (3600) 5.2, 4.9 / 5.1 / 5.8;  700 (4200) 5.8, 5.5 / 5.2 / 5.9
+//   64 + 2 x 8 of 128:   160 tokens (12800) 7.5, 7.2 / 5.4 / 5.5;  256 (20480) 10.5, 9.9 / 6.6 / 6.4
+// (4096 tokens of 16 + 2 x 4 heads of 256, 100 MB, 28.3: 3.6 TB/s).
 template <int D, int NH>
 __global__ __launch_bounds__(256) void attn_qk_kernel(const QkParams p) {
   constexpr int EPL = D / 64;  // elements per lane
@@ -1191,15 +1195,16 @@ extern "C" int gdn_attn_qk(const void* qg, int64_t qg_ld, const void* k_new, con
   p.eps = eps;
   p.log2_base = log2f(rope_base);
   hipStream_t st = static_cast<hipStream_t>(stream);
-  // heads per wave by the number of tokens (attn_qk_kernel's comment has both sides of each line)
+  // heads per wave by the rows of all heads (attn_qk_kernel's comment has both sides of each line)
   auto launch = [&](auto nh) {
     constexpr int NH = decltype(nh)::value;
     const dim3 grid(static_cast<unsigned>((B * T * ((Hq + 2 * Hkv + NH - 1) / NH) + 3) / 4));
     if (D == 256) hipLaunchKernelGGL((attn_qk_kernel<256, NH>), grid, dim3(256), 0, st, p);
     else hipLaunchKernelGGL((attn_qk_kernel<128, NH>), grid, dim3(256), 0, st, p);
   };
-  if (B * T <= 128) launch(std::integral_constant<int, 1>{});
-  else if (B * T < 512) launch(std::integral_constant<int, 3>{});
+  const int64_t rows = B * T * (Hq + 2 * Hkv);
+  if (rows <= 4096) launch(std::integral_constant<int, 1>{});
+  else if (rows <= 16384) launch(std::integral_constant<int, 3>{});
   else launch(std::integral_constant<int, 6>{});
   return gdn_host::check_launch("gdn_attn_qk");
 }

@@ -89,11 +89,17 @@ def test_qk_prep_matches_oracle():
 
 
 @pytest.mark.parametrize("B,T,Hq,Hkv,D,wdt", [
-    (1, 128, 10, 2, 256, torch.float32),   # one head a wave, its last size
-    (3, 43, 10, 2, 128, torch.bfloat16),   # 129 tokens: three heads a wave, 14 heads in 5 groups
+    (1, 128, 10, 2, 256, torch.float32),
+    (3, 43, 10, 2, 128, torch.bfloat16),
     (1, 511, 5, 1, 256, torch.float16),
-    (2, 256, 10, 2, 256, torch.bfloat16),  # 512 tokens: six heads a wave, the last with two
+    (1, 292, 10, 2, 256, torch.float32),   # 4088 rows of all heads: one head a wave, its last size
+    (1, 293, 10, 2, 256, torch.float16),   # 4102: three heads a wave, 14 heads in 5 groups
+    (2, 256, 10, 2, 256, torch.bfloat16),
     (1, 601, 4, 4, 128, torch.float32),
+    (1, 1170, 10, 2, 128, torch.float16),  # 16380: its last size
+    (1, 1171, 10, 2, 128, torch.bfloat16),  # 16394: six heads a wave, the last with two
+    (3, 391, 10, 2, 256, torch.float32),
+    (1, 1400, 4, 4, 128, torch.float32),
 ])
 def test_qk_prep_head_groups(B, T, Hq, Hkv, D, wdt):
     """The prep's head groups at their edges, with rows at an odd element
