@@ -176,10 +176,15 @@ CASES = {
     # 128-row tiles with keys split over workgroups: ranges without keys (row 0), one block
     # per range, a last tile of 8 rows; and more ranges than the combine takes in one pass
     "prefill_split_empty": (2, 130, [0, 700], 5, True),
-    "prefill_split_blocks": (1, 128, [2000], 33, True),
+    "prefill_split_blocks": (1, 128, [1984], 33, True),
     "prefill_split_d128": (1, 300, [333], 3, False, (16, 4, 128)),
-    "decode_split_70": (1, 1, [4500], 70, True),
+    "decode_split_70": (1, 1, [4479], 70, True),
 }
+
+
+def _filled_ranges(L, n_split):
+    """How many of n_split ranges hold keys: gdn_attn_fwd rounds their length up to whole 64-key blocks."""
+    return -(-L // (64 * -(-(-(-L // n_split)) // 64)))
 
 
 @pytest.mark.parametrize("name", list(CASES))
@@ -194,6 +199,8 @@ def test_attention_matches_oracle(name):
     Hq, Hkv, D = CASES[name][5] if len(CASES[name]) > 5 else (16, 4, 256)
     gen = torch.Generator().manual_seed(72)
     L = max(pos0) + T
+    if name in ("prefill_split_blocks", "decode_split_70"):
+        assert _filled_ranges(L, n_split) == n_split
     cap = L + 40
     kc = _bf16(gen, B, Hkv, cap, D)
     vc = _bf16(gen, B, Hkv, cap, D)
@@ -212,6 +219,22 @@ def test_attention_matches_oracle(name):
     got = _np(out)
     assert np.isfinite(got).all()
     assert _row_errs(got, ref).max() < ATT_TOL
+
+
+@pytest.mark.parametrize("D", [256, 128])
+@pytest.mark.parametrize("at", [4400, 100])
+def test_combine_of_two_passes_of_ranges_rescales(D, at):
+    """70 ranges of 64 keys, merged 64 in the first pass and 6 in the second, with a score of about 11 (the
+    others are about 1) in one key of either pass: the sums of the other pass are scaled down by e^-8 or so."""
+    gen = torch.Generator().manual_seed(86)
+    Hq, Hkv, L = 8, 2, 4480
+    assert _filled_ranges(L, 70) == 70
+    kc, vc, q = _bf16(gen, 1, Hkv, L, D), _bf16(gen, 1, Hkv, L, D), _bf16(gen, 1, 1, Hq, D)
+    kc[:, :, at] = q[:, 0, ::Hq // Hkv] * (11.0 / D ** 0.5)
+    out = att.attn_fwd(q.to(DEV), kc.to(DEV), vc.to(DEV), torch.tensor([L - 1], dtype=torch.int32, device=DEV), L,
+                       n_split=70)
+    ref = oa.attention(_np(q), _np(kc), _np(vc), [L - 1], D ** -0.5)
+    assert _row_errs(_np(out), ref).max() < ATT_TOL
 
 
 @pytest.mark.parametrize("T,n_split,heads", [(130, 1, (16, 4, 256)), (130, 2, (16, 4, 256)), (300, 1, (16, 4, 128))])
@@ -326,6 +349,30 @@ def test_decoder_layer_matches_oracle():
         ref = oa.decoder_layer(lp, _np(x), oc, _oracle_args(ARGS), round_fn=bf16_round)
         assert _row_errs(_np(y), ref).max() < LAYER_TOL
     assert cache.size() == 39 and cache.pos0.tolist() == [39, 39]
+
+
+@pytest.mark.parametrize("B,T,past", [(2, 1, 700), (1, 8, 1000), (1, 130, 900)])
+def test_attention_layer_splits_its_keys_and_matches_oracle(B, T, past):
+    """The layer's own choice of key ranges: 4 rows a kv-head (16-row tiles), 32 (64-row) and 520 (128-row)."""
+    torch.manual_seed(87)
+    gen = torch.Generator().manual_seed(87)
+    layer = mx.Attention(ARGS, device=DEV)
+    _randomise_norms(layer, gen)
+    Hq, Hkv, D, L = layer.Hq, layer.Hkv, layer.D, past + T
+    assert layer._splits(B, T, L) > 1
+    cache = mx.KVCache(B, Hkv, D, L, DEV)
+    cache.state = [_bf16(gen, B, Hkv, past, D).to(DEV) for _ in range(2)]
+    oc = oa.empty_cache(B, Hkv, L, D)
+    oc["k"][:, :, :past], oc["v"][:, :, :past] = (_np(t) for t in cache.state)
+    oc["offset"][:] = past
+    w = _np(layer.qkv_proj)
+    p = dict(q_proj=w[:2 * Hq * D], k_proj=w[2 * Hq * D:(2 * Hq + Hkv) * D], v_proj=w[(2 * Hq + Hkv) * D:],
+             o_proj=_np(layer.o_proj), q_norm=_np(layer.q_norm.weight), k_norm=_np(layer.k_norm.weight))
+    x = _bf16(gen, B, T, ARGS.hidden_size)
+    y = layer(x.to(DEV), cache)
+    ref = oa.attention_layer(p, _np(x), oc, _oracle_args(ARGS), round_fn=bf16_round)
+    assert _row_errs(_np(y), ref).max() < LAYER_TOL
+    assert cache.pos0.tolist() == [L] * B
 
 
 def test_mtp_head_matches_oracle_and_rolls_back():

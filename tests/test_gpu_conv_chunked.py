@@ -220,3 +220,77 @@ def test_masked_rows_equal_unfused(B, S, Hk, Hv, w_dtype, kind, with_cs):
                               t["cs"], mask=mask)
     _assert_equal(got, (y, s, cs))
     assert torch.isfinite(got[0].float()).all() and torch.isfinite(got[1]).all()
+
+
+def _masked_pair(t, Hk, Hv, mask, cu, idx=None, pools=(None, None)):
+    """The fused pass and the two launches on the same masked rows."""
+    q, k, v, cs = mx.gdn_conv_prologue(t["qkv"], t["w"], Hk, Hv, D, D, t["cs"], mask, cu_seqlens=cu)
+    y, s = mx.gated_delta_update(q, k, v, t["a"], t["b"], t["A_log"], t["dt_bias"],
+                                 t["state"] if idx is None else pools[1], mask, cu_seqlens=cu, chunked=True,
+                                 state_index=idx)
+    got = mx.gdn_conv_chunked(t["qkv"], t["w"], Hk, Hv, D, D, t["a"], t["b"], t["A_log"], t["dt_bias"],
+                              t["state"] if idx is None else pools[0], t["cs"], cu_seqlens=cu, state_index=idx,
+                              mask=mask)
+    return got, (y, s, cs)
+
+
+@pytest.mark.parametrize("with_cs", [True, False])
+@pytest.mark.parametrize("pooled", [False, True])
+@pytest.mark.parametrize("packed", [True, False])
+def test_masked_packed_and_pooled_rows_equal_unfused(packed, pooled, with_cs):
+    """A mask with packed sequences (lengths below the conv window and none at all among them, their first
+    and last tokens masked), with pooled states, and with both."""
+    Hk, Hv = 2, 4
+    lens = [2, 0, 68, 130, 1, 3] if packed else [150] * 3
+    n, total = len(lens), sum(lens)
+    at = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    t = _inputs(2080, 1 if packed else n, total if packed else 150, Hk, Hv, cs=with_cs, n_seqs=n)
+    gen = torch.Generator().manual_seed(2081)
+    mask = torch.rand(total, generator=gen) < 0.7
+    for start, length in zip(at, lens):
+        if length > 2:
+            mask[[start, start + length - 1]] = False
+    mask = mask.view(t["qkv"].shape[:2]).to(DEV)
+    t["qkv"][~mask] = float("nan")
+    pool = (torch.randn(8, Hv, D, D, generator=gen) * 0.02).to(DEV)
+    idx = torch.tensor([4, 0, 2, 7, 1, 6][:n], dtype=torch.int32, device=DEV) if pooled else None
+    pools = (pool.clone(), pool.clone())
+    got, want = _masked_pair(t, Hk, Hv, mask, at.tolist() if packed else None, idx, pools)
+    _assert_equal(got, want)
+    assert torch.isfinite(got[0].float()).all() and torch.isfinite(got[1]).all()
+    if pooled:
+        left = [i for i in range(8) if i not in idx.tolist()]
+        assert torch.equal(pools[0][left], pool[left])
+
+
+@pytest.mark.parametrize("pooled", [False, True])
+def test_mixer_masked_prefill_takes_the_fused_path_and_matches_unfused(pooled):
+    """The layer on left-padded prompts, with dense and with pooled states, against the same layer with the
+    prologue launched on its own."""
+    m = mx.GatedDeltaNet(256, 2, 4, D, D, device=DEV)
+    m.reset_parameters(torch.Generator().manual_seed(2090))
+    gen = torch.Generator().manual_seed(2091)
+    x = torch.randn(3, 100, 256, generator=gen).to(torch.bfloat16).to(DEV)
+    mask = (torch.arange(100)[None, :] >= torch.tensor([[0], [37], [98]])).to(DEV)
+    cs = torch.randn(3, 3, m.conv_dim, generator=gen).to(torch.bfloat16).to(DEV)
+    states = (torch.randn(3, 4, D, D, generator=gen) * 0.02).to(DEV)
+    outs = []
+    with torch.no_grad():
+        for fused in (True, False):
+            c = mx.ArraysCache()
+            c[0] = cs.clone()
+            if pooled:
+                pool = mx.StatePool(5, 4, D, D, device=DEV)
+                slots = pool.alloc(5)
+                pool.release(slots[:1] + slots[3:4])
+                c[1] = mx.PooledBatch(pool, [slots[i] for i in (4, 1, 2)])
+                pool.scatter(c[1].slots, states)
+            else:
+                c[1] = states.clone()
+            if fused:
+                assert m._fused_prefill(m._project(x)[0], mask)
+            else:
+                m._fused_prefill = lambda qkv, mask: False
+            y = m(x, mask, c)
+            outs.append((y, c[1].pool.gather(c[1].slots) if pooled else c[1], c[0]))
+    _assert_equal(*outs)
