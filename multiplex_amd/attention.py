@@ -135,9 +135,10 @@ def attn_qk(qg: torch.Tensor, k_new: torch.Tensor, v_new: torch.Tensor, q_norm_w
     if q_out is None:
         q_out = torch.empty(B, T, Hq, D, dtype=torch.bfloat16, device=dev)
     qn, kn = q_norm_w.contiguous(), k_norm_w.contiguous()
-    _lib.call("gdn_attn_qk", _ptr(qg), qg_ld, _ptr(k_new), _ptr(v_new), kv_ld, _ptr(qn), _ptr(kn),
-              _dtype_code(qn, "q_norm_w"), float(eps), _ptr(pos0), _ptr(q_out), _ptr(k_cache), _ptr(v_cache),
-              B, T, Hq, Hkv, D, cap, int(rot), float(rope_base), _stream(dev))
+    with _on_device(dev):
+        _lib.call("gdn_attn_qk", _ptr(qg), qg_ld, _ptr(k_new), _ptr(v_new), kv_ld, _ptr(qn), _ptr(kn),
+                  _dtype_code(qn, "q_norm_w"), float(eps), _ptr(pos0), _ptr(q_out), _ptr(k_cache), _ptr(v_cache),
+                  B, T, Hq, Hkv, D, cap, int(rot), float(rope_base), _stream(dev))
     return q_out
 
 
@@ -193,9 +194,10 @@ def attn_fwd(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, pos0
         workspace = torch.empty(need, dtype=torch.uint8, device=dev)
     q = q.contiguous()
     scale = D ** -0.5 if scale is None else scale
-    _lib.call("gdn_attn_fwd", _ptr(q), _ptr(gate), qg_ld, _ptr(k_cache), _ptr(v_cache), _ptr(pos0), _ptr(out),
-              float(scale), B, T, Hq, Hkv, D, cap, int(kv_len_max), int(n_split), _ptr(workspace),
-              0 if workspace is None else workspace.numel() * workspace.element_size(), _stream(dev))
+    with _on_device(dev):
+        _lib.call("gdn_attn_fwd", _ptr(q), _ptr(gate), qg_ld, _ptr(k_cache), _ptr(v_cache), _ptr(pos0), _ptr(out),
+                  float(scale), B, T, Hq, Hkv, D, cap, int(kv_len_max), int(n_split), _ptr(workspace),
+                  0 if workspace is None else workspace.numel() * workspace.element_size(), _stream(dev))
     return out
 
 
@@ -227,8 +229,9 @@ def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float, *, residual: Opt
         residual = residual.contiguous()
         h = torch.empty_like(x)
     w = weight.contiguous()
-    _lib.call("gdn_rms_norm", _ptr(x), _ptr(residual), _ptr(h), _ptr(w), _dtype_code(w, "weight"), _ptr(out), y_ld,
-              rows, D, float(eps), _stream(dev))
+    with _on_device(dev):
+        _lib.call("gdn_rms_norm", _ptr(x), _ptr(residual), _ptr(h), _ptr(w), _dtype_code(w, "weight"), _ptr(out), y_ld,
+                  rows, D, float(eps), _stream(dev))
     return out if residual is None else (h, out)
 
 
@@ -239,7 +242,8 @@ def silu_mul(gate_up: torch.Tensor) -> torch.Tensor:
     I = gate_up.shape[-1] // 2
     gate_up = gate_up.contiguous()
     out = torch.empty(*gate_up.shape[:-1], I, dtype=gate_up.dtype, device=dev)
-    _lib.call("gdn_silu_mul", _ptr(gate_up), _ptr(out), gate_up.numel() // (2 * I), I, _stream(dev))
+    with _on_device(dev):
+        _lib.call("gdn_silu_mul", _ptr(gate_up), _ptr(out), gate_up.numel() // (2 * I), I, _stream(dev))
     return out
 
 

@@ -454,7 +454,8 @@ class PreparedRecurrent:
         if stream is not None:
             args = _lib.RecurrentArgs.from_buffer_copy(self._args)
             args.stream = _stream_handle(stream)
-        st = self._lib.gdn_recurrent(_lib.ctypes.byref(args))
+        with _on_device(self.device):
+            st = self._lib.gdn_recurrent(_lib.ctypes.byref(args))
         if st != _lib.OK:
             _lib.check("gdn_recurrent", st)
 
@@ -533,7 +534,8 @@ class PreparedCall:
 
     def launch(self, stream=None):
         args = self._args if stream is None else self._args[:-1] + (_stream_handle(stream),)
-        st = self._fn(*args)
+        with _on_device(self.device):
+            st = self._fn(*args)
         if st != _lib.OK:
             _lib.check(self._fn_name, st)
 
@@ -553,7 +555,8 @@ class PreparedChunked(PreparedCall):
 
     def _issue(self, fn, name, stream):
         args = self._args if stream is None else self._args[:-1] + (_stream_handle(stream),)
-        st = fn(*args)
+        with _on_device(self.device):
+            st = fn(*args)
         if st != _lib.OK:
             _lib.check(name, st)
 

@@ -99,8 +99,9 @@ def _launch(x, gate, norm_weight, eps, head_dim, weight, out, workspace):
     need = linear_decode_workspace_bytes(M, N, K)
     ws = (workspace if workspace is not None else DecodeWorkspace()).get(need, dev)
     nw_dt = _dtype_code(norm_weight, "norm_weight") if norm_weight is not None else 0
-    _lib.call("gdn_linear_decode", _ptr(x), ldx, _ptr(gate), ldg, _ptr(norm_weight), nw_dt, float(eps),
-              int(head_dim), _ptr(weight), _ptr(out), ldo, M, N, K, _ptr(ws), ws.numel(), _stream(dev))
+    with _on_device(dev):
+        _lib.call("gdn_linear_decode", _ptr(x), ldx, _ptr(gate), ldg, _ptr(norm_weight), nw_dt, float(eps),
+                  int(head_dim), _ptr(weight), _ptr(out), ldo, M, N, K, _ptr(ws), ws.numel(), _stream(dev))
     return out
 
 

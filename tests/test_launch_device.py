@@ -13,7 +13,19 @@ import pytest
 import torch
 
 import multiplex_amd as mx
-from multiplex_amd import _lib, attention, gated_delta, linear
+from multiplex_amd import _lib, attention, epilogue, gated_delta, linear
+
+
+class _Library:
+    """The library, with every launch given to ``call`` by its name."""
+
+    def __init__(self, call):
+        self._call = call
+
+    def __getattr__(self, name):
+        if name.endswith("_workspace_bytes"):
+            return lambda *sizes: 64
+        return lambda *args: self._call(name, *args)
 
 
 @pytest.fixture
@@ -30,9 +42,11 @@ def launches(monkeypatch):
     def call(name, *args):
         assert inside, f"{name} is launched on whichever device is current"
         made.append(name)
+        return _lib.OK
 
     monkeypatch.setattr(_lib, "call", call)
-    for mod in (attention, linear):
+    monkeypatch.setattr(_lib, "load", lambda: _Library(call))
+    for mod in (attention, epilogue, gated_delta, linear):
         monkeypatch.setattr(mod, "_on_device", enter, raising=False)
         monkeypatch.setattr(mod, "_stream", lambda dev: 0)
         monkeypatch.setattr(mod, "_require_device", lambda tensors, names: torch.device("cpu"))
@@ -73,3 +87,34 @@ def test_projection_of_few_rows(launches):
     x, w = torch.zeros(3, 1, 512, dtype=torch.bfloat16), torch.zeros(2056, 512, dtype=torch.bfloat16)
     assert linear._rows16(x, w, 3).shape == (3, 1, 2056)
     assert launches == ["gdn_linear_rows16"]
+
+
+def _bf16(*shape):
+    return torch.zeros(*shape, dtype=torch.bfloat16)
+
+
+def test_attention_launches(launches):
+    cache = _bf16(2, 1, 64, 128)
+    pos0 = torch.zeros(2, dtype=torch.int32)
+    q = attention.attn_qk(_bf16(2, 1, 512), _bf16(2, 1, 128), _bf16(2, 1, 128), _bf16(128), _bf16(128), 1e-6, pos0,
+                          cache, cache.clone(), 32, 1e7)
+    attention.attn_fwd(q, cache, cache, pos0, 4)
+    attention.rms_norm(_bf16(3, 64), _bf16(64), 1e-6)
+    attention.silu_mul(_bf16(3, 64))
+    assert launches == ["gdn_attn_qk", "gdn_attn_fwd", "gdn_rms_norm", "gdn_silu_mul"]
+
+
+def test_epilogue_and_decode_projection_launches(launches):
+    epilogue.gated_rms_norm(_bf16(3, 128), _bf16(3, 128))
+    linear.linear_decode(_bf16(3, 512), _bf16(8, 512))
+    linear.gated_norm_linear_decode(_bf16(3, 512), _bf16(3, 512), None, 1e-6, 128, _bf16(8, 512))
+    assert launches == ["gdn_gated_rmsnorm", "gdn_linear_decode", "gdn_linear_decode"]
+
+
+def test_prepared_launches(launches):
+    gated_delta.PreparedCall("gdn_x", (0,), {}, (), torch.device("cpu")).launch()
+    chunked = gated_delta.PreparedChunked("gdn_chunk_fwd", (0,), {}, (), torch.device("cpu"))
+    chunked.launch_prep()
+    chunked.launch_scan(7)
+    gated_delta.PreparedRecurrent(_lib.RecurrentArgs(), {}, torch.device("cpu")).launch(7)
+    assert launches == ["gdn_x", "gdn_chunk_prep", "gdn_chunk_scan", "gdn_recurrent"]
