@@ -479,21 +479,23 @@ class Attention(torch.nn.Module):
         if self._cus is None:
             self._cus = torch.cuda.get_device_properties(self.qkv_proj.device).multi_processor_count
         rows = T * (self.Hq // self.Hkv)
-        if rows >= 512:
-            n = B * self.Hkv * -(-rows // 128)
-            tile = 128
-            ranges = max(1, min(self._cus // n, (L - T) // 256))
-        elif rows <= 16:
+        n = B * self.Hkv
+        if rows <= 16:
             tile = 16
-            n = B * self.Hkv
-            ranges = max(1, min(round(self._cus / n), max(self._cus // n, L // 512), L // 64 - 1))
-        else:
-            n = B * self.Hkv * -(-rows // 64)
+            ranges = min(round(self._cus / n), max(self._cus // n, L // 512), L // 64 - 1)
+        elif rows < 512:
             tile = 64
-            ranges = max(1, min(self._cus // n, L // 128), min(2 * self._cus // n, L // 256))
+            n *= -(-rows // 64)
+            ranges = max(min(self._cus // n, L // 128), min(2 * self._cus // n, L // 256))
+        else:
+            tile = 128
+            n *= -(-rows // 128)
+            ranges = min(self._cus // n, (L - T) // 256)
+        if ranges <= 1:
+            return 1
         blocks = -(-L // 64)
-        of_range = max(1, -(-(-(-L // ranges)) // 64))  # as gdn_attn_fwd takes it
-        ranges = max(1, -(-blocks // of_range))
+        of_range = -(-L // (64 * ranges))  # as gdn_attn_fwd takes it
+        ranges = -(-blocks // of_range)
         block_us, mb_us = _SPLIT_US[tile][self.D > 128]
         partials = 4e-6 * B * self.Hkv * rows * ranges * self.D  # MB
         return ranges if block_us * (blocks - of_range) > 3.5 + mb_us * partials else 1

@@ -155,11 +155,12 @@ def _stream(dev: torch.device) -> int:
 
 
 _HERE = contextlib.nullcontext()
+_current_device = getattr(torch._C, "_cuda_getDevice", None) or torch.cuda.current_device
 
 
 def _on_device(dev: torch.device):
     """``torch.cuda.device(dev)``, or nothing to enter where it is current."""
-    return _HERE if dev.index == torch.cuda.current_device() else torch.cuda.device(dev)
+    return _HERE if dev.index == _current_device() else torch.cuda.device(dev)
 
 
 def _mask_u8(mask: Optional[torch.Tensor], shape, what="mask") -> Optional[torch.Tensor]:

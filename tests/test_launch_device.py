@@ -54,7 +54,7 @@ def launches(monkeypatch):
 
 
 def test_on_device_enters_another_device_only(monkeypatch):
-    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    monkeypatch.setattr(gated_delta, "_current_device", lambda: 0)
     assert isinstance(gated_delta._on_device(torch.device("cuda", 0)), contextlib.nullcontext)
     other = gated_delta._on_device(torch.device("cuda", 1))
     assert isinstance(other, torch.cuda.device) and other.idx == 1
