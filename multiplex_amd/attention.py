@@ -480,6 +480,8 @@ class Attention(torch.nn.Module):
             self._cus = torch.cuda.get_device_properties(self.qkv_proj.device).multi_processor_count
         rows = T * (self.Hq // self.Hkv)
         n = B * self.Hkv
+        if n == 0:
+            return 1
         if rows <= 16:
             tile = 16
             ranges = min(round(self._cus / n), max(self._cus // n, L // 512), L // 64 - 1)

@@ -22,6 +22,12 @@ def test_every_range_holds_keys_and_lies_on_whole_blocks(Hq, Hkv, D):
     assert layer._splits(1, 0, 0) == 1
 
 
+@pytest.mark.parametrize("T", [1, 8, 200])
+def test_a_batch_of_no_rows_takes_one_range(T):
+    """(All of its requests have left.)"""
+    assert _ranges(16, 4, 256, [(0, T, T), (0, T, 5000)]) == {(0, T, T): 1, (0, T, 5000): 1}
+
+
 def _ranges(Hq, Hkv, D, calls):
     layer = mx.Attention(mx.AttentionArgs(64, Hq, Hkv, D, 64), device="cpu")
     layer._cus = 256

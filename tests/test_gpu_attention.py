@@ -375,6 +375,16 @@ def test_attention_layer_splits_its_keys_and_matches_oracle(B, T, past):
     assert cache.pos0.tolist() == [L] * B
 
 
+@pytest.mark.parametrize("T", [1, 5, 130])
+def test_attention_layer_of_no_rows(T):
+    """A batch whose requests have all left: no output rows, and the cache advances."""
+    layer = mx.Attention(ARGS, device=DEV)
+    cache = mx.KVCache(2, layer.Hkv, layer.D, 300, DEV)
+    cache.filter([])
+    y = layer(torch.empty(0, T, ARGS.hidden_size, dtype=torch.bfloat16, device=DEV), cache)
+    assert y.shape == (0, T, ARGS.hidden_size) and cache.batch == 0 and cache.pos0.numel() == 0
+
+
 def test_mtp_head_matches_oracle_and_rolls_back():
     """MTPHead (mtp.py:181-194): a 4-position call from an empty draft cache,
     two draft steps, then a trim back to the committed length and the same
