@@ -5,12 +5,15 @@ Loading fails loudly: there is no CPU or eager fallback behind this module.
 
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import os
 import struct
 import threading
 from ctypes import POINTER, Structure, c_char_p, c_float, c_int, c_int32, c_int64, c_size_t, c_void_p
 from pathlib import Path
+
+import torch
 
 LIB_PATH = Path(__file__).resolve().parent / "libgdn.so"
 
@@ -248,17 +251,37 @@ def check(fn: str, status: int) -> None:
     raise GDNError(fn, status, msg)
 
 
-def call(name: str, *args) -> None:
-    status = getattr(_lib if _lib is not None else load(), name)(*args)
+# A device's default stream is handle 0, and a launch on handle 0 runs on the
+# current device: every launch is made with its tensors' device current.
+_current_device = getattr(torch._C, "_cuda_getDevice", None) or torch.cuda.current_device
+_HERE = contextlib.nullcontext()
+
+
+def on_device(device: torch.device):
+    """``torch.cuda.device(device)``, or nothing to enter where it is current."""
+    return _HERE if device.index == _current_device() else torch.cuda.device(device)
+
+
+def call(device: torch.device, name: str, *args) -> None:
+    """The library's function ``name`` with ``device`` current."""
+    if device.index != _current_device():
+        with torch.cuda.device(device):
+            status = getattr(load(), name)(*args)
+    else:
+        status = getattr(_lib if _lib is not None else load(), name)(*args)
     if status != OK:
         check(name, status)
 
 
-def call_recurrent(*fields) -> None:
+def call_recurrent(device: torch.device, *fields) -> None:
     """``gdn_recurrent`` with the values of :class:`RecurrentArgs` in field
     order (0 for a null pointer)."""
     if _lib is None:
         load()
-    status = _recurrent(_RECURRENT.pack(*fields))
+    if device.index != _current_device():
+        with torch.cuda.device(device):
+            status = _recurrent(_RECURRENT.pack(*fields))
+    else:
+        status = _recurrent(_RECURRENT.pack(*fields))
     if status != OK:
         check("gdn_recurrent", status)

@@ -36,7 +36,7 @@ from typing import List, Optional, Sequence
 import torch
 
 from . import _lib
-from .gated_delta import _dtype_code, _on_device, _ptr, _require_device, _stream
+from .gated_delta import _dtype_code, _ptr, _require_device, _stream
 from .linear import linear
 
 __all__ = [
@@ -117,10 +117,11 @@ def attn_qk(qg: torch.Tensor, k_new: torch.Tensor, v_new: torch.Tensor, q_norm_w
     caches ``[B, Hkv, cap, D]``; pos0 ``[B]`` int32 device offsets.
     Returns q ``[B, T, Hq, D]``.
     """
-    dev = _require_device([qg, k_new, v_new, q_norm_w, k_norm_w, pos0, k_cache, v_cache],
-                          ["qg", "k_new", "v_new", "q_norm_w", "k_norm_w", "pos0", "k_cache", "v_cache"])
-    for t, n in ((qg, "qg"), (k_new, "k_new"), (v_new, "v_new"), (k_cache, "k_cache"), (v_cache, "v_cache")):
-        _bf16(t, n)
+    dev = _require_device((qg, k_new, v_new, q_norm_w, k_norm_w, pos0, k_cache, v_cache),
+                          ("qg", "k_new", "v_new", "q_norm_w", "k_norm_w", "pos0", "k_cache", "v_cache"))
+    if not qg.dtype is k_new.dtype is v_new.dtype is k_cache.dtype is v_cache.dtype is torch.bfloat16:
+        for t, n in ((qg, "qg"), (k_new, "k_new"), (v_new, "v_new"), (k_cache, "k_cache"), (v_cache, "v_cache")):
+            _bf16(t, n)
     B, Hkv, cap, D = k_cache.shape
     if v_cache.shape != k_cache.shape or not k_cache.is_contiguous() or not v_cache.is_contiguous():
         raise ValueError("k_cache and v_cache must be contiguous [B, Hkv, cap, D] tensors of one shape")
@@ -130,15 +131,14 @@ def attn_qk(qg: torch.Tensor, k_new: torch.Tensor, v_new: torch.Tensor, q_norm_w
     kv_ld = _token_stride(k_new, Hkv * D, "k_new")
     if _token_stride(v_new, Hkv * D, "v_new") != kv_ld:
         raise ValueError("k_new and v_new must share one token stride")
-    if pos0.dtype != torch.int32 or tuple(pos0.shape) != (B,):
+    if pos0.dtype != torch.int32 or pos0.shape != (B,):
         raise ValueError(f"pos0 must be int32 [{B}]")
     if q_out is None:
         q_out = torch.empty(B, T, Hq, D, dtype=torch.bfloat16, device=dev)
     qn, kn = q_norm_w.contiguous(), k_norm_w.contiguous()
-    with _on_device(dev):
-        _lib.call("gdn_attn_qk", _ptr(qg), qg_ld, _ptr(k_new), _ptr(v_new), kv_ld, _ptr(qn), _ptr(kn),
-                  _dtype_code(qn, "q_norm_w"), float(eps), _ptr(pos0), _ptr(q_out), _ptr(k_cache), _ptr(v_cache),
-                  B, T, Hq, Hkv, D, cap, int(rot), float(rope_base), _stream(dev))
+    _lib.call(dev, "gdn_attn_qk", _ptr(qg), qg_ld, _ptr(k_new), _ptr(v_new), kv_ld, _ptr(qn), _ptr(kn),
+              _dtype_code(qn, "q_norm_w"), float(eps), _ptr(pos0), _ptr(q_out), _ptr(k_cache), _ptr(v_cache),
+              B, T, Hq, Hkv, D, cap, int(rot), float(rope_base), _stream(dev))
     return q_out
 
 
@@ -161,19 +161,19 @@ def _check_attn_fwd(q, k_cache, v_cache, pos0, kv_len_max, gate, out):
         raise ValueError(f"caches [{Bc}, {Hkv}, {cap}, {Dc}] do not match q's batch {B} and head dim {D}")
     if Hkv == 0 or Hq % Hkv != 0:
         raise ValueError(f"Hq={Hq} is not a multiple of Hkv={Hkv}")
-    if not isinstance(pos0, torch.Tensor) or pos0.dtype != torch.int32 or tuple(pos0.shape) != (B,):
+    if not isinstance(pos0, torch.Tensor) or pos0.dtype != torch.int32 or pos0.shape != (B,):
         raise ValueError(f"pos0 must be an int32 tensor of shape [{B}]")
     if not T <= int(kv_len_max) <= cap:
         raise ValueError(f"kv_len_max={kv_len_max} must lie in [T={T}, cap={cap}]")
     qg_ld = 0
     if gate is not None:
         _bf16(gate, "gate")
-        if gate.dim() != 3 or tuple(gate.shape[:2]) != (B, T):
+        if gate.dim() != 3 or gate.shape[:2] != (B, T):
             raise ValueError(f"gate must be [B={B}, T={T}, {Hq * 2 * D}]")
         qg_ld = _token_stride(gate, Hq * 2 * D, "gate")
     if out is not None:
         _bf16(out, "out")
-        if tuple(out.shape) != (B, T, Hq, D) or not out.is_contiguous():
+        if out.shape != (B, T, Hq, D) or not out.is_contiguous():
             raise ValueError(f"out must be a contiguous [{B}, {T}, {Hq}, {D}] tensor")
     return B, T, Hq, D, Hkv, cap, qg_ld
 
@@ -186,18 +186,17 @@ def attn_fwd(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, pos0
     (``[B, T, Hq*2D]``, the q_proj output) when given.  ``kv_len_max`` bounds
     ``pos0[b] + T`` (host value; keys beyond it are not read)."""
     B, T, Hq, D, Hkv, cap, qg_ld = _check_attn_fwd(q, k_cache, v_cache, pos0, kv_len_max, gate, out)
-    dev = _require_device([q, k_cache, v_cache, pos0, gate, out], ["q", "k_cache", "v_cache", "pos0", "gate", "out"])
+    dev = _require_device((q, k_cache, v_cache, pos0, gate, out), ("q", "k_cache", "v_cache", "pos0", "gate", "out"))
     if out is None:
         out = torch.empty(B, T, Hq, D, dtype=torch.bfloat16, device=dev)
-    need = int(_lib.load().gdn_attn_workspace_bytes(B, T, Hq, Hkv, D, n_split))
+    need = int(_lib.load().gdn_attn_workspace_bytes(B, T, Hq, Hkv, D, n_split)) if n_split != 1 else 0
     if need > 0 and (workspace is None or workspace.numel() * workspace.element_size() < need):
         workspace = torch.empty(need, dtype=torch.uint8, device=dev)
     q = q.contiguous()
     scale = D ** -0.5 if scale is None else scale
-    with _on_device(dev):
-        _lib.call("gdn_attn_fwd", _ptr(q), _ptr(gate), qg_ld, _ptr(k_cache), _ptr(v_cache), _ptr(pos0), _ptr(out),
-                  float(scale), B, T, Hq, Hkv, D, cap, int(kv_len_max), int(n_split), _ptr(workspace),
-                  0 if workspace is None else workspace.numel() * workspace.element_size(), _stream(dev))
+    _lib.call(dev, "gdn_attn_fwd", _ptr(q), _ptr(gate), qg_ld, _ptr(k_cache), _ptr(v_cache), _ptr(pos0), _ptr(out),
+              float(scale), B, T, Hq, Hkv, D, cap, int(kv_len_max), int(n_split), _ptr(workspace),
+              0 if workspace is None else workspace.numel() * workspace.element_size(), _stream(dev))
     return out
 
 
@@ -229,9 +228,8 @@ def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float, *, residual: Opt
         residual = residual.contiguous()
         h = torch.empty_like(x)
     w = weight.contiguous()
-    with _on_device(dev):
-        _lib.call("gdn_rms_norm", _ptr(x), _ptr(residual), _ptr(h), _ptr(w), _dtype_code(w, "weight"), _ptr(out), y_ld,
-                  rows, D, float(eps), _stream(dev))
+    _lib.call(dev, "gdn_rms_norm", _ptr(x), _ptr(residual), _ptr(h), _ptr(w), _dtype_code(w, "weight"), _ptr(out),
+              y_ld, rows, D, float(eps), _stream(dev))
     return out if residual is None else (h, out)
 
 
@@ -242,8 +240,7 @@ def silu_mul(gate_up: torch.Tensor) -> torch.Tensor:
     I = gate_up.shape[-1] // 2
     gate_up = gate_up.contiguous()
     out = torch.empty(*gate_up.shape[:-1], I, dtype=gate_up.dtype, device=dev)
-    with _on_device(dev):
-        _lib.call("gdn_silu_mul", _ptr(gate_up), _ptr(out), gate_up.numel() // (2 * I), I, _stream(dev))
+    _lib.call(dev, "gdn_silu_mul", _ptr(gate_up), _ptr(out), gate_up.numel() // (2 * I), I, _stream(dev))
     return out
 
 
@@ -347,8 +344,8 @@ class KVCache:
         p = self.pos0
         if not p.is_cuda or p.dtype is not torch.int32 or not p.is_contiguous() or not -2**31 <= delta < 2**31:
             return False
-        with _on_device(p.device):
-            _lib.call("gdn_pos_add", p.data_ptr(), p.numel(), delta, lo, _stream(p.device))
+        dev = p.device
+        _lib.call(dev, "gdn_pos_add", p.data_ptr(), p.numel(), delta, lo, _stream(dev))
         return True
 
     def filter(self, keep: Sequence[int]) -> None:
@@ -506,9 +503,7 @@ class Attention(torch.nn.Module):
         B, T, _ = x.shape
         Hq, Hkv, D = self.Hq, self.Hkv, self.D
         qkv = linear(x, self.qkv_proj)
-        qg = qkv[..., : 2 * Hq * D]
-        k = qkv[..., 2 * Hq * D : (2 * Hq + Hkv) * D]
-        v = qkv[..., (2 * Hq + Hkv) * D :]
+        qg, k, v = qkv.split((2 * Hq * D, Hkv * D, Hkv * D), -1)
         cache.reserve(T)
         q = attn_qk(qg, k, v, self.q_norm.weight, self.k_norm.weight, self.args.rms_norm_eps, cache.pos0,
                     cache.keys, cache.values, self.args.rot, self.args.rope_theta)

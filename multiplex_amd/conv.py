@@ -16,7 +16,7 @@ import torch
 
 from . import _lib
 from .gated_delta import (CHUNK, IntSeq, PreparedCall, _addr, _contig, _cu_seqlens, _dtype_code, _gate_codes, _gate_pair,
-                          _int_rows, _mask_u8, _on_device, _param_codes, _ptr, _require_device, _state_operands, _stream,
+                          _int_rows, _mask_u8, _param_codes, _ptr, _require_device, _state_operands, _stream,
                           _token_rows)
 
 __all__ = ["gdn_conv_prologue", "prepare_conv_prologue", "conv_state_commit", "gdn_conv_chunked",
@@ -114,8 +114,7 @@ def gdn_conv_prologue(qkv: torch.Tensor, conv_weight: torch.Tensor, num_k_heads:
     """
     args, _keep, outs, dev = _prologue_args(qkv, conv_weight, num_k_heads, num_v_heads, head_k_dim, head_v_dim,
                                             conv_state, mask, cu_seqlens, eps, write_conv_state, conv_state_out)
-    with _on_device(dev):
-        _lib.call("gdn_conv_prologue", *args)
+    _lib.call(dev, "gdn_conv_prologue", *args)
     return outs
 
 
@@ -158,9 +157,8 @@ def conv_state_commit(conv_state: Optional[torch.Tensor], qkv: torch.Tensor, n_c
     ld = _token_rows(qkv, C)
     if ld is None:
         qkv, ld = qkv.contiguous(), C
-    with _on_device(dev):
-        _lib.call("gdn_conv_state_commit", _ptr(conv_state), _ptr(qkv), io, ld, _ptr(m), _ptr(n), _ptr(out),
-                  B, T, C, Kt, _stream(dev))
+    _lib.call(dev, "gdn_conv_state_commit", _ptr(conv_state), _ptr(qkv), io, ld, _ptr(m), _ptr(n), _ptr(out),
+              B, T, C, Kt, _stream(dev))
     return out
 
 
@@ -242,8 +240,7 @@ def gdn_conv_chunked(qkv: torch.Tensor, conv_weight: torch.Tensor, num_k_heads: 
     args, _keep, outs, dev = _conv_chunked_args(qkv, conv_weight, num_k_heads, num_v_heads, head_k_dim,
                                                 head_v_dim, a, b, A_log, dt_bias, state, conv_state, cu_seqlens,
                                                 eps, state_out, workspace, state_index, write_conv_state, mask)
-    with _on_device(dev):
-        _lib.call("gdn_chunk_fwd_conv_masked", *args)
+    _lib.call(dev, "gdn_chunk_fwd_conv_masked", *args)
     return outs
 
 
@@ -291,10 +288,9 @@ def gdn_conv_decode(qkv, conv_weight, num_k_heads, num_v_heads, head_k_dim, head
     y = torch.empty(B, 1, Hv, D, dtype=bf16, device=dev)
     new_state = torch.empty(B, Hv, D, D, dtype=torch.float32, device=dev)
     cs_out = torch.empty(B, 3, C, dtype=bf16, device=dev) if write_conv_state else None
-    with _on_device(dev):
-        _lib.call("gdn_conv_decode", qkv_p, ld, w_p, cs_p, _addr(cs_out), float(eps), a.data_ptr(), b.data_ptr(), la,
-                  A_log.data_ptr(), dt_bias.data_ptr(), _dtype_code(A_log, "A_log"), st_p, y.data_ptr(),
-                  new_state.data_ptr(), B, Hk, Hv, D, D, _stream(dev))
+    _lib.call(dev, "gdn_conv_decode", qkv_p, ld, w_p, cs_p, _addr(cs_out), float(eps), a.data_ptr(), b.data_ptr(), la,
+              A_log.data_ptr(), dt_bias.data_ptr(), _dtype_code(A_log, "A_log"), st_p, y.data_ptr(),
+              new_state.data_ptr(), B, Hk, Hv, D, D, _stream(dev))
     return y, new_state, cs_out
 
 

@@ -15,7 +15,7 @@ from typing import Optional
 import torch
 
 from . import _lib
-from .gated_delta import PreparedCall, _dtype_code, _on_device, _ptr, _require_device, _stream
+from .gated_delta import PreparedCall, _dtype_code, _ptr, _require_device, _stream
 
 __all__ = ["gated_rms_norm", "prepare_gated_rms_norm"]
 
@@ -84,8 +84,7 @@ def gated_rms_norm(x: torch.Tensor, gate: torch.Tensor, weight: Optional[torch.T
     apart, as a fused in_proj output gives); it is then read in place.
     """
     args, _, out, dev = _norm_args(x, gate, weight, eps, out)
-    with _on_device(dev):
-        _lib.call("gdn_gated_rmsnorm", *args)
+    _lib.call(dev, "gdn_gated_rmsnorm", *args)
     return out
 
 

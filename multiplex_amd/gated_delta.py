@@ -19,7 +19,6 @@ Every tensor must live on one ROCm device; there is no CPU path.
 
 from __future__ import annotations
 
-import contextlib
 from typing import Optional, Sequence, Union
 
 import torch
@@ -152,15 +151,6 @@ def _stream(dev: torch.device) -> int:
     if _raw_stream is not None and dev.index is not None:
         return _raw_stream(dev.index)
     return torch.cuda.current_stream(dev).cuda_stream
-
-
-_HERE = contextlib.nullcontext()
-_current_device = getattr(torch._C, "_cuda_getDevice", None) or torch.cuda.current_device
-
-
-def _on_device(dev: torch.device):
-    """``torch.cuda.device(dev)``, or nothing to enter where it is current."""
-    return _HERE if dev.index == _current_device() else torch.cuda.device(dev)
 
 
 def _mask_u8(mask: Optional[torch.Tensor], shape, what="mask") -> Optional[torch.Tensor]:
@@ -424,12 +414,11 @@ def _recurrent(q, k, v, gx, gy, gate_mode, A_log, dt_bias, state, mask, *,
     snaps = (torch.empty(sh.B, sh.T, sh.Hv, sh.Dv, sh.Dk, dtype=torch.float32, device=dev)
              if snapshots else None)
     commit = None if commit_len is None else _int_rows(commit_len, n_rows, dev, "commit_len")
-    with _on_device(dev):
-        _lib.call_recurrent(
-            _addr(q), k.data_ptr(), v.data_ptr(), qkv_code, gate_mode, gx.data_ptr(), gy.data_ptr(), gate_code,
-            param_code, _addr(A_log), _addr(dt_bias), _addr(state), _addr(out_state), _addr(snaps), _addr(y_t),
-            _addr(mask_u8), _addr(cu), _addr(commit), _addr(idx), n_rows, sh.T, sh.Hk, sh.Hv, sh.Dk, sh.Dv, n_slots,
-            g_ld, _stream(dev), int(y_from))
+    _lib.call_recurrent(
+        dev, _addr(q), k.data_ptr(), v.data_ptr(), qkv_code, gate_mode, gx.data_ptr(), gy.data_ptr(), gate_code,
+        param_code, _addr(A_log), _addr(dt_bias), _addr(state), _addr(out_state), _addr(snaps), _addr(y_t),
+        _addr(mask_u8), _addr(cu), _addr(commit), _addr(idx), n_rows, sh.T, sh.Hk, sh.Hv, sh.Dk, sh.Dv, n_slots,
+        g_ld, _stream(dev), int(y_from))
     return y_t, out_state, snaps
 
 
@@ -455,7 +444,7 @@ class PreparedRecurrent:
         if stream is not None:
             args = _lib.RecurrentArgs.from_buffer_copy(self._args)
             args.stream = _stream_handle(stream)
-        with _on_device(self.device):
+        with _lib.on_device(self.device):
             st = self._lib.gdn_recurrent(_lib.ctypes.byref(args))
         if st != _lib.OK:
             _lib.check("gdn_recurrent", st)
@@ -535,7 +524,7 @@ class PreparedCall:
 
     def launch(self, stream=None):
         args = self._args if stream is None else self._args[:-1] + (_stream_handle(stream),)
-        with _on_device(self.device):
+        with _lib.on_device(self.device):
             st = self._fn(*args)
         if st != _lib.OK:
             _lib.check(self._fn_name, st)
@@ -556,7 +545,7 @@ class PreparedChunked(PreparedCall):
 
     def _issue(self, fn, name, stream):
         args = self._args if stream is None else self._args[:-1] + (_stream_handle(stream),)
-        with _on_device(self.device):
+        with _lib.on_device(self.device):
             st = fn(*args)
         if st != _lib.OK:
             _lib.check(name, st)
@@ -606,8 +595,7 @@ def _chunked(q, k, v, gx, gy, gate_mode, A_log, dt_bias, state, *, cu_seqlens=No
     args, _keep, y_t, out_state, dev = _chunk_args(q, k, v, gx, gy, gate_mode, A_log, dt_bias, state,
                                                    cu_seqlens=cu_seqlens, state_out=state_out,
                                                    workspace=workspace, state_index=state_index, mask=mask)
-    with _on_device(dev):
-        _lib.call("gdn_chunk_fwd", *args)
+    _lib.call(dev, "gdn_chunk_fwd", *args)
     return y_t, out_state
 
 

@@ -33,7 +33,7 @@ import torch
 import torch.autograd.forward_ad as forward_ad
 
 from . import _lib
-from .gated_delta import _dtype_code, _on_device, _ptr, _require_device, _stream
+from .gated_delta import _dtype_code, _ptr, _require_device, _stream
 
 __all__ = ["linear", "DECODE_MAX_ROWS", "FUSED_NORM_MAX_ROWS", "DecodeWorkspace", "linear_decode",
            "gated_norm_linear_decode", "linear_decode_workspace_bytes", "decode_shape_ok"]
@@ -99,9 +99,8 @@ def _launch(x, gate, norm_weight, eps, head_dim, weight, out, workspace):
     need = linear_decode_workspace_bytes(M, N, K)
     ws = (workspace if workspace is not None else DecodeWorkspace()).get(need, dev)
     nw_dt = _dtype_code(norm_weight, "norm_weight") if norm_weight is not None else 0
-    with _on_device(dev):
-        _lib.call("gdn_linear_decode", _ptr(x), ldx, _ptr(gate), ldg, _ptr(norm_weight), nw_dt, float(eps),
-                  int(head_dim), _ptr(weight), _ptr(out), ldo, M, N, K, _ptr(ws), ws.numel(), _stream(dev))
+    _lib.call(dev, "gdn_linear_decode", _ptr(x), ldx, _ptr(gate), ldg, _ptr(norm_weight), nw_dt, float(eps),
+              int(head_dim), _ptr(weight), _ptr(out), ldo, M, N, K, _ptr(ws), ws.numel(), _stream(dev))
     return out
 
 
@@ -117,10 +116,10 @@ def linear(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     rows = x.numel() // K if K else 0
     if (_rows16_shape(rows, N, K) and x.dtype is torch.bfloat16 and weight.dtype is torch.bfloat16
             and x.is_cuda and weight.is_cuda and x.shape[-1] == K and not _needs_operator(x, weight)
-            and x.is_contiguous() and weight.is_contiguous() and x.device == weight.device):
+            and x.is_contiguous() and weight.is_contiguous() and x.get_device() == weight.get_device()):
         xp, wp = x.data_ptr(), weight.data_ptr()
-        if xp % 16 == 0 and wp % 16 == 0:
-            return _rows16(x, weight, rows)
+        if (xp | wp) % 16 == 0:
+            return _rows16(x, xp, wp, rows, N, K)
     return torch.nn.functional.linear(x, weight)
 
 
@@ -170,12 +169,10 @@ def _rows16_shape(rows, N, K) -> bool:
     return 1 <= rows <= most and 512 <= K <= 12288 and K % _K_SLICE == 0 and 2048 < N <= _MAX_COLUMNS and N % 8 == 0
 
 
-def _rows16(x, weight, rows):
-    N, K = weight.shape
+def _rows16(x, x_addr, w_addr, rows, N, K):
     dev = x.device
     out = torch.empty(*x.shape[:-1], N, dtype=torch.bfloat16, device=dev)
-    with _on_device(dev):
-        _lib.call("gdn_linear_rows16", x.data_ptr(), K, weight.data_ptr(), out.data_ptr(), N, rows, N, K, _stream(dev))
+    _lib.call(dev, "gdn_linear_rows16", x_addr, K, w_addr, out.data_ptr(), N, rows, N, K, _stream(dev))
     return out
 
 

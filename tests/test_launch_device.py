@@ -13,7 +13,7 @@ import pytest
 import torch
 
 import multiplex_amd as mx
-from multiplex_amd import _lib, attention, epilogue, gated_delta, linear
+from multiplex_amd import _lib, attention, conv, epilogue, gated_delta, linear
 
 
 class _Library:
@@ -25,12 +25,12 @@ class _Library:
     def __getattr__(self, name):
         if name.endswith("_workspace_bytes"):
             return lambda *sizes: 64
-        return lambda *args: self._call(name, *args)
+        return lambda *args: self._call(name)
 
 
 @pytest.fixture
 def launches(monkeypatch):
-    """The names of the library calls made, each inside its device's context."""
+    """The names of the launches made, each with its tensors' device current, which device 0 is before."""
     inside, made = [], []
 
     @contextlib.contextmanager
@@ -39,24 +39,25 @@ def launches(monkeypatch):
         yield
         inside.pop()
 
-    def call(name, *args):
+    def call(name):
         assert inside, f"{name} is launched on whichever device is current"
         made.append(name)
         return _lib.OK
 
-    monkeypatch.setattr(_lib, "call", call)
-    monkeypatch.setattr(_lib, "load", lambda: _Library(call))
-    for mod in (attention, epilogue, gated_delta, linear):
-        monkeypatch.setattr(mod, "_on_device", enter, raising=False)
+    monkeypatch.setattr(_lib, "_current_device", lambda: 0)
+    monkeypatch.setattr(torch.cuda, "device", enter)
+    monkeypatch.setattr(_lib, "_lib", _Library(call))
+    monkeypatch.setattr(_lib, "_recurrent", lambda packed: call("gdn_recurrent"))
+    for mod in (attention, conv, epilogue, gated_delta, linear):
         monkeypatch.setattr(mod, "_stream", lambda dev: 0)
         monkeypatch.setattr(mod, "_require_device", lambda tensors, names: torch.device("cpu"))
     return made
 
 
 def test_on_device_enters_another_device_only(monkeypatch):
-    monkeypatch.setattr(gated_delta, "_current_device", lambda: 0)
-    assert isinstance(gated_delta._on_device(torch.device("cuda", 0)), contextlib.nullcontext)
-    other = gated_delta._on_device(torch.device("cuda", 1))
+    monkeypatch.setattr(_lib, "_current_device", lambda: 0)
+    assert isinstance(_lib.on_device(torch.device("cuda", 0)), contextlib.nullcontext)
+    other = _lib.on_device(torch.device("cuda", 1))
     assert isinstance(other, torch.cuda.device) and other.idx == 1
 
 
@@ -85,7 +86,7 @@ def test_cache_offsets(launches):
 
 def test_projection_of_few_rows(launches):
     x, w = torch.zeros(3, 1, 512, dtype=torch.bfloat16), torch.zeros(2056, 512, dtype=torch.bfloat16)
-    assert linear._rows16(x, w, 3).shape == (3, 1, 2056)
+    assert linear._rows16(x, x.data_ptr(), w.data_ptr(), 3, 2056, 512).shape == (3, 1, 2056)
     assert launches == ["gdn_linear_rows16"]
 
 
@@ -118,3 +119,19 @@ def test_prepared_launches(launches):
     chunked.launch_scan(7)
     gated_delta.PreparedRecurrent(_lib.RecurrentArgs(), {}, torch.device("cpu")).launch(7)
     assert launches == ["gdn_x", "gdn_chunk_prep", "gdn_chunk_scan", "gdn_recurrent"]
+
+
+def test_gated_delta_and_conv_launches(launches, monkeypatch):
+    q, v = _bf16(1, 64, 1, 128), _bf16(1, 64, 1, 128)
+    gates, par = _bf16(1, 64, 1), torch.zeros(1)
+    state = torch.zeros(1, 1, 128, 128)
+    for chunked in (False, True):
+        gated_delta.gated_delta_update(q, q, v, gates, gates, par, par, state, chunked=chunked)
+    qkv, w = _bf16(1, 64, 384), _bf16(384, 4)
+    conv.gdn_conv_prologue(qkv, w, 1, 1, 128, 128)
+    conv.gdn_conv_chunked(qkv, w, 1, 1, 128, 128, gates, gates, par, par)
+    assert conv.gdn_conv_decode(qkv[:, :1], w, 1, 1, 128, 128, gates[:, :1], gates[:, :1], par, par, None, None)
+    monkeypatch.setattr(conv, "_int_rows", lambda rows, n, dev, what: rows)
+    conv.conv_state_commit(None, qkv[:, :4], torch.tensor([2], dtype=torch.int32))
+    assert launches == ["gdn_recurrent", "gdn_chunk_fwd", "gdn_conv_prologue", "gdn_chunk_fwd_conv_masked",
+                        "gdn_conv_decode", "gdn_conv_state_commit"]
