@@ -12,13 +12,15 @@ Graph-replayed against the separate norm kernel plus hipBLASLt at hidden
 2048, the fused norm + out_proj takes 7.4-8.1 us against 12.6-13.4 us up to
 16 rows, and loses beyond (11.4 against 10.9 us at 32 rows, 16.4 against
 13.1 us at 64).  So the mixer uses ``gated_norm_linear_decode`` up to
-``FUSED_NORM_MAX_ROWS`` rows; ``linear_decode`` (the same kernel without the
-norm) is the unfused reference for tests.
+``FUSED_NORM_MAX_ROWS`` rows; ``linear_decode`` (the same call without the
+norm) is the unfused reference for tests.  Up to 16 rows and above 2048
+columns it runs ``gdn_linear_rows16``'s kernel, which leaves the workspace it
+is given alone.
 
-:func:`linear` is the layers' plain projection: up to 16 rows
+:func:`linear` is the layers' plain projection: a few rows by
 ``gdn_linear_rows16``, the library beyond.
 
-The kernel sums its K slices through a workspace of fp32 partials and one
+The sliced kernel sums its K slices through a workspace of fp32 partials and one
 ticket per output tile; the tickets must start at zero and every call
 leaves them zero, so one zero-initialised workspace serves every call of a
 module on one stream (calls that overlap, on several streams, need one
