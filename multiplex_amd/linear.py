@@ -126,17 +126,20 @@ def linear(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
 
 
 _transform_level = getattr(torch._C._functorch, "maybe_current_level", None)
+_dispatch_modes = getattr(torch._C, "_len_torch_dispatch_stack", None)
 
 
 def _needs_operator(x, weight) -> bool:
     """Whether something follows or replaces the operator on these operands: a
     recorded gradient, a forward-mode tangent (its tensors are plain ones that
-    ask for no gradient), a function transform (vmap, jvp, grad), autocast, a
-    tensor subclass."""
+    ask for no gradient), a function transform (vmap, jvp, grad), a dispatch
+    mode or a trace, autocast, a tensor subclass."""
     if (type(x) is not torch.Tensor or type(weight) not in (torch.Tensor, torch.nn.Parameter)
             or torch.is_autocast_enabled() or (torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad))):
         return True
     if _transform_level is None or _transform_level() is not None:
+        return True
+    if _dispatch_modes is None or _dispatch_modes() or torch.jit.is_tracing():
         return True
     # (outside a dual level, -1, no tensor has a tangent)
     return getattr(forward_ad, "_current_level", 0) >= 0 and any(

@@ -5,6 +5,8 @@ from __future__ import annotations
 import pytest
 import torch
 import torch.autograd.forward_ad as fwad
+from torch.fx.experimental.proxy_tensor import make_fx
+from torch.utils.flop_counter import FlopCounterMode
 
 from multiplex_amd import linear
 
@@ -48,6 +50,28 @@ def test_function_transforms_need_the_operator(transform):
     else:
         torch.func.vmap(f)(w[None])
     assert seen == [True]
+
+
+@pytest.mark.parametrize("trace", ["make_fx", "jit", "flops"])
+def test_traces_and_dispatch_modes_need_the_operator(trace):
+    """Their operands may be plain tensors that hold real values."""
+    x, w = _operands()
+    seen = []
+
+    def f(x, w):
+        seen.append(linear._needs_operator(x, w))
+        return torch.nn.functional.linear(x, w)
+
+    if trace == "make_fx":
+        make_fx(f, tracing_mode="real")(x, w)
+    elif trace == "jit":
+        torch.jit.trace(f, (x, w), check_trace=False)
+    else:
+        with FlopCounterMode(display=False):
+            f(x, w)
+    assert seen == [True]
+    with torch.device("cpu"):  # a mode for new tensors only
+        assert not linear._needs_operator(x, w)
 
 
 @pytest.mark.parametrize("rows,N,K,taken", [
