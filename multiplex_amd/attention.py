@@ -246,6 +246,11 @@ def silu_mul(gate_up: torch.Tensor) -> torch.Tensor:
 
 # ------------------------------------------------------------------ cache
 
+def _pos_add(pos0: torch.Tensor, delta: int, lo: int) -> None:
+    dev = pos0.device
+    _lib.call(dev, "gdn_pos_add", pos0.data_ptr(), pos0.numel(), delta, lo, _stream(dev))
+
+
 class KVCache:
     """One attention layer's KV cache, ``[B, Hkv, capacity, D]`` bf16.
 
@@ -339,13 +344,14 @@ class KVCache:
         return n
 
     def _pos_add(self, delta: int, lo: int) -> bool:
-        """``pos0 = max(pos0 + delta, lo)`` in one launch (``gdn_pos_add``), or
-        False for offsets the kernel does not take (e.g. on the host)."""
+        """``pos0 = max(pos0 + delta, lo)`` in one launch, or False for offsets
+        the kernel does not take (on the host, or without memory of their own:
+        fake and other subclassed tensors)."""
         p = self.pos0
-        if not p.is_cuda or p.dtype is not torch.int32 or not p.is_contiguous() or not -2**31 <= delta < 2**31:
+        if (type(p) is not torch.Tensor or not p.is_cuda or p.dtype is not torch.int32 or not p.is_contiguous()
+                or not -2**31 <= delta < 2**31):
             return False
-        dev = p.device
-        _lib.call(dev, "gdn_pos_add", p.data_ptr(), p.numel(), delta, lo, _stream(dev))
+        _pos_add(p, delta, lo)
         return True
 
     def filter(self, keep: Sequence[int]) -> None:
