@@ -461,11 +461,13 @@ class Attention(torch.nn.Module):
         tiles' workgroups, one per CU, times the ranges fit the CUs, each at
         least 256 keys of the prefix (512 tokens over 4096: 122 -> 55; 128
         over 8192: 212 -> 39; 1024 over none stays whole: 38, two ranges 43).
-        Up to 16 rows (decode, draft verify): one workgroup per CU, 128 or
-        more keys (one token over 1024: 30.3 -> 11.4; of four over 4001:
-        120 -> 19.6), or about one of 512 or more.  Between: 64-row tiles, two workgroups per CU; at
-        least 128 keys up to one workgroup per CU and 256 beyond (8 tokens
-        over 16384: 828 -> 31; 32 over 1024: 53 -> 16; 64 over 8192: 417 -> 40).
+        Up to 16 rows (decode, draft verify): at most one workgroup per CU,
+        of 128 keys or more, or the number nearest to one per CU where it
+        leaves 512 keys each (one token over 1024: 30.3 -> 11.4; four rows
+        over 4001: 120 -> 19.6).  Between: 64-row tiles, two workgroups per
+        CU; at least 128 keys up to one workgroup per CU and 256 beyond (8
+        tokens over 16384: 828 -> 31; 32 over 1024: 53 -> 16; 64 over 8192:
+        417 -> 40).
 
         The blocks that a workgroup's chain is then shorter by have to pay
         for the partial results, which are written, read and merged

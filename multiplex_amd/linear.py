@@ -161,9 +161,10 @@ def _rows16_shape(rows, N, K) -> bool:
         with the weight in the cache at 75, by 57% at most (K = 2560 at 4608 to 6144 columns)
       K to 8192, 4 rows:   4096 x 8192 15.5 / 12.4, 15.5 / 13.0; 12288 x 8192 35.3 / 29.6, 39.5 / 31.4
       K to 12288, 2 rows:  4096 x 12288 18.4 / 16.2, 21.0 / 17.0; 16384 x 12288 69.9 / 69.1, 82.4 / 86.4
-      K over 4096 at 4104 to 8192 columns, whose tiles load the CUs unevenly or (8192 wide) are read
-        7168 to 16384 bytes apart, is the library's: 5120 x 5120 at 4 rows 14.5 / 13.0, 14.0 / 11.5;
-        6144 x 8192 23.2 / 19.3, 21.4 / 17.9; 8192 x 8192 32.0 / 20.3, 28.9 / 21.7
+      K over 4096 at 4104 to 8192 columns, where the busiest CU has two 16-column tiles and most have
+        fewer, is the library's: 5120 x 5120 at 4 rows 14.5 / 13.0, 14.0 / 11.5; 6144 x 8192 23.2 / 19.3,
+        21.4 / 17.9 (and, with two on every CU, 8192 x 8192 32.0 / 20.3, 28.9 / 21.7; 8192 x 6144, 21% faster
+        than the library from memory, goes there with them)
     """
     if K <= 4096:
         most = 16
